@@ -1,0 +1,8 @@
+// The tile attention kernel (pfa_tile_attn.h) for f32 inputs.
+#include "pfa_tile_attn.h"
+
+namespace pfa {
+int tile_attn_launch_f32(const AttnArgs& a, int out_dtype, int D, hipStream_t s) {
+  return tile::launch<PFA_F32>(a, out_dtype, D, s);
+}
+}  // namespace pfa

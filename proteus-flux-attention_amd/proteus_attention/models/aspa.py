@@ -1745,17 +1745,24 @@ class AdaptiveSparseAttention(nn.Module):
                             quantized=use_quant, candidates=True, structured=True)
             self._last_shortlist_backend_info = get_last_backend_info()
             return
+        # A window over the whole sequence takes every key 0..t, whatever
+        # anchors and prototypes add: the implicit causal branch attends the
+        # same sets on MFMA tiles, with no candidate lists to build or gather.
+        causal = local_w >= T and L >= T
         sets = None
         row_batch = None
-        if K > 0:
+        if K > 0 and not causal:
             sets = _sa._proto_prefix_sets(self._last_token_similarity, K)
             if B > 1:
                 # rows past a device row count hold arbitrary values: clamp
                 # them into range (the builder does not read those rows)
                 rh = row_head.clamp(0, heads.numel() - 1) if rows_dev is not None else row_head
                 row_batch = (heads.index_select(0, rh) // H).to(torch.int32)
-        cand, lens = _sa._shortlist_build_device(token_idx, row_batch, T, L, local_w, stride, slots, sets,
-                                                 n_rows_dev=rows_dev)
+        if causal:
+            cand, lens = None, (token_idx + 1 if self.record_shortlist_lengths else None)
+        else:
+            cand, lens = _sa._shortlist_build_device(token_idx, row_batch, T, L, local_w, stride, slots, sets,
+                                                     n_rows_dev=rows_dev)
         self._last_shortlist_lengths = lens
         out4 = _hip.tensor4(attn.view(B, T, H, D), H, "bthd")
         if use_quant:
@@ -1766,12 +1773,12 @@ class AdaptiveSparseAttention(nn.Module):
             scales = self._quantize_qkv(q5, B, T, heads, q8)
             _sa._attn_launch(_hip.tensor4(q8[:, :, 0], H, "bthd"), _hip.tensor4(q8[:, :, 1], H, "bthd"),
                              _hip.tensor4(q8[:, :, 2], H, "bthd"), torch.int8, out4, qkv.dtype, H, T, D, token_idx,
-                             row_head, heads, cand, lens, None, None, 1.0 / math.sqrt(D),
+                             row_head, heads, cand, None if causal else lens, None, None, 1.0 / math.sqrt(D),
                              (scales[0], scales[1], scales[2]), device, n_rows_dev=rows_dev)
         else:
             _sa._attn_launch(_hip.tensor4(q5[:, :, 0], H, "bthd"), _hip.tensor4(q5[:, :, 1], H, "bthd"),
                              _hip.tensor4(q5[:, :, 2], H, "bthd"), qkv.dtype, out4, qkv.dtype, H, T, D, token_idx,
-                             row_head, heads, cand, lens, None, None, 1.0 / math.sqrt(D), (None, None, None), device,
+                             row_head, heads, cand, None if causal else lens, None, None, 1.0 / math.sqrt(D), (None, None, None), device,
                              n_rows_dev=rows_dev)
         _record_backend("hip", device=str(device), tokens=T, rows=int(token_idx.numel()), L=L,
                         quantized=use_quant, candidates=True, structured=False)
