@@ -474,6 +474,19 @@ int pfa_quantize_heads_int8(pfa_tensor4 x, int dtype, int H, int64_t T, int D,
                             pfa_tensor4 dst, int dst_dtype, float* scales,
                             void* workspace, size_t ws_bytes, void* stream);
 
+/* pfa_quantize_heads_int8 of q, k and v (same sizes, head list and mode) in
+ * the same launches.  scales: (3, n_heads), n_heads = all (b, h) heads; the
+ * workspace is sized by pfa_quantize_heads_workspace_size for 3 * P_cap. */
+int pfa_quantize_qkv_int8(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, int dtype,
+                          int H, int n_heads, int64_t T, int D,
+                          const int32_t* head_map, int P_cap,
+                          const int32_t* summary, int mode, float percentile,
+                          double ema_decay, float* ema_q, float* ema_k,
+                          float* ema_v, int valid_q, int valid_k, int valid_v,
+                          pfa_tensor4 dst_q, pfa_tensor4 dst_k,
+                          pfa_tensor4 dst_v, int dst_dtype, float* scales,
+                          void* workspace, size_t ws_bytes, void* stream);
+
 /* Per compact head, the largest token among its packed rows (needed by the
  * explicit-mask branch: sparse_attn.py:1010-1015). */
 int pfa_head_max_token(const int32_t* token_idx, const int32_t* row_offsets,

@@ -57,6 +57,7 @@ EXPORTED_SYMBOLS = (
     "pfa_head_max_token",
     "pfa_quantize_heads_workspace_size",
     "pfa_quantize_heads_int8",
+    "pfa_quantize_qkv_int8",
     "pfa_rope_qk_inplace",
     "pfa_rope_k_inplace",
     "pfa_rope_k_zero_inplace",
@@ -140,6 +141,9 @@ _SIGNATURES = {
     "pfa_quantize_heads_workspace_size": ([_i32, _i64, _i32, _i32, ctypes.POINTER(_sz)], _i32),
     "pfa_quantize_heads_int8": ([Tensor4, _i32, _i32, _i64, _i32, _vp, _i32, _vp, _i32, _f32, ctypes.c_double, _vp,
                                  _i32, Tensor4, _i32, _vp, _vp, _sz, _vp], _i32),
+    "pfa_quantize_qkv_int8": ([Tensor4, Tensor4, Tensor4, _i32, _i32, _i32, _i64, _i32, _vp, _i32, _vp, _i32, _f32,
+                               ctypes.c_double, _vp, _vp, _vp, _i32, _i32, _i32, Tensor4, Tensor4, Tensor4, _i32, _vp,
+                               _vp, _sz, _vp], _i32),
     "pfa_rope_qk_inplace": ([_vp, _i32, _i32, _i64, _i32, _i32, _vp, _vp, _vp], _i32),
     "pfa_rope_k_inplace": ([_vp, _i32, _i32, _i64, _i32, _i32, _vp, _vp, _vp], _i32),
     "pfa_rope_k_zero_inplace": ([_vp, _i32, _i32, _i64, _i32, _i32, _vp, _vp, _vp, _vp], _i32),

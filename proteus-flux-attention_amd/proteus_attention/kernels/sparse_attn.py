@@ -565,6 +565,39 @@ def quantize_heads_int8(
     _hip.check(rc, "pfa_quantize_heads_int8")
 
 
+def quantize_qkv_int8(
+    x4s: Tuple["_hip.Tensor4", "_hip.Tensor4", "_hip.Tensor4"],
+    dtype: torch.dtype,
+    H: int,
+    T: int,
+    D: int,
+    head_map: Optional[torch.Tensor],
+    P_cap: int,
+    mode: str,
+    percentile: float,
+    ema_decay: float,
+    emas: Tuple[Optional[torch.Tensor], Optional[torch.Tensor], Optional[torch.Tensor]],
+    ema_valid: Tuple[bool, bool, bool],
+    dst4s: Tuple["_hip.Tensor4", "_hip.Tensor4", "_hip.Tensor4"],
+    dst_dtype: torch.dtype,
+    scales: torch.Tensor,
+    device: torch.device,
+) -> None:
+    """quantize_heads_int8 of q, k and v in the same launches; scales is
+    (3, B*H) f32."""
+
+    lib = _hip.lib()
+    m = _QUANT_MODES[mode]
+    ws = _workspace(_size_out(lib.pfa_quantize_heads_workspace_size, 3 * int(P_cap), int(T), int(D), m), device)
+    with _hip.TIMER.timed("quantize_heads_int8"):
+        rc = lib.pfa_quantize_qkv_int8(*x4s, _hip.dtype_tag(dtype), int(H), int(scales.size(1)), int(T), int(D),
+                                       _hip.ptr(head_map), int(P_cap), None, m, float(percentile), float(ema_decay),
+                                       *(_hip.ptr(e) for e in emas), *(1 if v else 0 for v in ema_valid), *dst4s,
+                                       _hip.dtype_tag(dst_dtype), _hip.ptr(scales), _hip.ptr(ws), ws.numel(),
+                                       _hip.stream_ptr(device))
+    _hip.check(rc, "pfa_quantize_qkv_int8")
+
+
 def aspa_sparse_attention(
     q: torch.Tensor,
     k: torch.Tensor,

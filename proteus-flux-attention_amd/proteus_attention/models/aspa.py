@@ -759,20 +759,24 @@ class AdaptiveSparseAttention(nn.Module):
         active heads of one of q/k/v, with this module's mode and its
         per-head EMA buffer (re-initialised when P changes, as the
         reference's is)."""
-        mode = self.quantize_sparse_int8_mode
-        ema, valid = None, False
-        if mode == "ema_percentile":
-            ema = getattr(self, ema_buffer)
-            valid = bool(ema is not None and ema.numel() == P and self._quant_ema_flags.get(ema_buffer, False)
-                         and ema.device == scales.device and ema.dtype == torch.float32)
-            if not valid:
-                ema = torch.empty(P, dtype=torch.float32, device=scales.device)
-        _sa.quantize_heads_int8(x4, dtype, H, T, D, head_map, P, summary, mode,
+        ema, valid = self._quant_ema(ema_buffer, P, scales.device)
+        _sa.quantize_heads_int8(x4, dtype, H, T, D, head_map, P, summary, self.quantize_sparse_int8_mode,
                                 float(self.quantize_sparse_int8_percentile), float(self.quantize_sparse_int8_ema_decay),
                                 ema, valid, dst4, dst_dtype, scales, scales.device)
         if ema is not None:
             setattr(self, ema_buffer, ema)
             self._quant_ema_flags[ema_buffer] = True
+
+    def _quant_ema(self, name: str, P: int, device: torch.device) -> Tuple[Optional[torch.Tensor], bool]:
+        """The EMA buffer `name` for P heads and whether it holds values
+        ("ema_percentile" mode; a new buffer when it does not fit)."""
+        if self.quantize_sparse_int8_mode != "ema_percentile":
+            return None, False
+        ema = getattr(self, name)
+        if (ema is not None and ema.numel() == P and self._quant_ema_flags.get(name, False)
+                and ema.device == device and ema.dtype == torch.float32):
+            return ema, True
+        return torch.empty(P, dtype=torch.float32, device=device), False
 
     # ------------------------------------------------------------------
     # device stages
@@ -1792,9 +1796,18 @@ class AdaptiveSparseAttention(nn.Module):
         H, D = self.h_total, self.d_head
         P = int(heads.numel())
         scales = torch.empty(3, B * H, dtype=torch.float32, device=q5.device)
-        for i, name in enumerate(("_quant_ema_q", "_quant_ema_k", "_quant_ema_v")):
-            self._quantize_heads(_hip.tensor4(q5[:, :, i], H, "bthd"), q5.dtype, H, T, D, heads, P, None,
-                                 _hip.tensor4(dst5[:, :, i], H, "bthd"), dst5.dtype, scales[i], name)
+        names = ("_quant_ema_q", "_quant_ema_k", "_quant_ema_v")
+        emas = [self._quant_ema(n, P, scales.device) for n in names]
+        _sa.quantize_qkv_int8(tuple(_hip.tensor4(q5[:, :, i], H, "bthd") for i in range(3)), q5.dtype, H, T, D, heads, P,
+                              self.quantize_sparse_int8_mode, float(self.quantize_sparse_int8_percentile),
+                              float(self.quantize_sparse_int8_ema_decay), tuple(e for e, _ in emas),
+                              tuple(v for _, v in emas),
+                              tuple(_hip.tensor4(dst5[:, :, i], H, "bthd") for i in range(3)), dst5.dtype, scales,
+                              q5.device)
+        for n, (e, _) in zip(names, emas):
+            if e is not None:
+                setattr(self, n, e)
+                self._quant_ema_flags[n] = True
         return scales
 
     def _router_regulariser(self, gate_probs: torch.Tensor) -> Optional[torch.Tensor]:
