@@ -504,6 +504,26 @@ def _mfma_causal_ok(dtype: torch.dtype, D: int, *t4s: "_hip.Tensor4") -> bool:
     return True
 
 
+# Implicit causal bf16 rows on the tile kernel (pfa_sparse_attn_fwd) rather
+# than the structured kernel (pfa_shortlist_attn_fwd with a full window), by
+# the number of 64-row blocks.  The tile kernel splits keys over its waves when
+# the blocks do not fill the chip and keeps P at 16 more bits; the structured
+# kernel's larger blocks win once they do.  Measured on one box (us, structured
+# / tile):
+#   D = 64:  129 blocks, T 8,192: 160 / 68; 512, T 4,096: 76 / 63; 1,024, T 8,192:
+#            172 / 155; 2,048, T 2,048: 96 / 109; 4,096, T 32,768: 1,985 / 2,108
+#   D = 32:  129 blocks, T 8,192: 159 / 63; 2,048, T 4,096: 158 / 136; 4,096,
+#            T 32,768: 1,811 / 1,563
+#   D = 128: 129 blocks, T 8,192: 195 / 153; 254, T 4,096: 99 / 77; 511, T 4,096:
+#            118 / 132
+_CAUSAL_TILE_BLOCKS = {16: None, 32: None, 64: 1024, 128: 256}
+
+
+def _causal_tiles(rows: int, D: int) -> bool:
+    most = _CAUSAL_TILE_BLOCKS.get(int(D), 0)
+    return most is None or (int(rows) + 63) // 64 <= most
+
+
 def _causal_attn_mfma(q4, k4, v4, out4, H: int, T: int, D: int, token_idx: torch.Tensor, row_head: torch.Tensor,
                       head_map: Optional[torch.Tensor], device: torch.device) -> None:
     """Implicit-causal attention (row r attends to keys 0..token_idx[r] of its
@@ -719,8 +739,9 @@ def aspa_sparse_attention(
     H = batch_heads
     scale = 1.0 / math.sqrt(head_dim)
     t4 = (_hip.tensor4(qc, H), _hip.tensor4(kc, H), _hip.tensor4(vc, H), _hip.tensor4(out, H))
-    if (cand is None and causal_mask is None and not is_quantized and out_dtype == q.dtype
-            and _mfma_causal_ok(q.dtype, head_dim, *t4)):
+    causal_bf16 = (cand is None and causal_mask is None and not is_quantized and out_dtype == q.dtype
+                   and _mfma_causal_ok(q.dtype, head_dim, *t4))
+    if causal_bf16 and not _causal_tiles(n_rows, head_dim):
         # implicit causal branch on MFMA tiles (rows are packed by (head, token))
         _causal_attn_mfma(*t4, H, tokens, head_dim, token_idx, row_head, None, device)
         _record_backend("hip", device=str(device), heads=batch_heads, tokens=tokens, max_rows=int(max_rows),
@@ -729,8 +750,11 @@ def aspa_sparse_attention(
     _attn_launch(_hip.tensor4(qc, H), _hip.tensor4(kc, H), _hip.tensor4(vc, H), q.dtype, _hip.tensor4(out, H),
                  out_dtype, H, tokens, head_dim, token_idx, row_head, None, cand, lens, causal_mask, head_max, scale,
                  scales, device)
-    _record_backend("hip", device=str(device), heads=batch_heads, tokens=tokens, max_rows=int(max_rows),
-                    quantized=bool(is_quantized), candidates=cand is not None)
+    details = dict(device=str(device), heads=batch_heads, tokens=tokens, max_rows=int(max_rows),
+                   quantized=bool(is_quantized), candidates=cand is not None)
+    if causal_bf16:
+        details["mfma"] = True
+    _record_backend("hip", **details)
     return out
 
 

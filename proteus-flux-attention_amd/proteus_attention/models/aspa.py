@@ -526,6 +526,10 @@ class AdaptiveSparseAttention(nn.Module):
     # schedules (aspa.py:731-930, 1037-1173) -- host arithmetic
     # ------------------------------------------------------------------
     def _choose_active_k(self, seq_len: int) -> int:
+        self._last_target_k = self._active_k(seq_len)
+        return self._last_target_k
+
+    def _active_k(self, seq_len: int) -> int:
         if seq_len <= self.seq_low:
             target = self.h_active_max
         elif seq_len >= self.seq_high:
@@ -535,9 +539,7 @@ class AdaptiveSparseAttention(nn.Module):
             if self.h_active_curve != 1.0:
                 ratio = max(0.0, min(1.0, ratio)) ** self.h_active_curve
             target = int(math.floor(self.h_active_max - ratio * (self.h_active_max - self.h_active_min) + 1e-6))
-        target = max(self.h_active_min, min(target, self.h_active_max))
-        self._last_target_k = target
-        return target
+        return max(self.h_active_min, min(target, self.h_active_max))
 
     def _nucleus_head_count(self, head_probs: torch.Tensor, target_p: float, max_cap: int) -> int:
         if max_cap <= 1:
@@ -1024,7 +1026,8 @@ class AdaptiveSparseAttention(nn.Module):
         out4 = out.view(B, T, H, D)
         t4 = (_hip.tensor4(q5[:, :, 0], H, "bthd"), _hip.tensor4(q5[:, :, 1], H, "bthd"),
               _hip.tensor4(q5[:, :, 2], H, "bthd"), _hip.tensor4(out4, H, "bthd"))
-        if out.dtype == qkv.dtype and _sa._mfma_causal_ok(qkv.dtype, D, *t4):
+        if (out.dtype == qkv.dtype and _sa._mfma_causal_ok(qkv.dtype, D, *t4)
+                and not _sa._causal_tiles(int(token_idx.numel()), D)):
             # flash-style causal tiles on MFMA (64 queries x 64 keys); rows
             # past the device count carry token -1, which the kernel skips
             _sa._causal_attn_mfma(*t4, H, T, D, token_idx, row_head, head_map, qkv.device)
@@ -1189,7 +1192,7 @@ class AdaptiveSparseAttention(nn.Module):
             if self.token_keep_threshold > 0.0:
                 return False
             sims = bool(self.proto_enabled and self.routing_prototypes is not None)
-            if self._shortlist_plan(B, T, self._compute_cvt_alpha(T), x.dtype, sims=sims)["structured"]:
+            if self._shortlist_plan(B, T, self._compute_cvt_alpha(T), x.dtype, sims=sims)["fits"]:
                 return False
         return True
 
@@ -1641,10 +1644,15 @@ class AdaptiveSparseAttention(nn.Module):
         anchors = stride > 0 and slots > 0
         w_eff = max(1, local_w)
         bound = w_eff + ((min(slots, (T - 1) // stride) + 1) if anchors else 0) + K
-        structured = (dtype == torch.bfloat16 and D in _sa.STRUCTURED_HEAD_DIMS and bound <= L and K <= 1024
-                      and not _hip.env_flag("PFA_FORCE_GENERIC"))
+        fits = (dtype == torch.bfloat16 and D in _sa.STRUCTURED_HEAD_DIMS and bound <= L and K <= 1024
+                and not _hip.env_flag("PFA_FORCE_GENERIC"))
+        # a window over the whole sequence is implicitly causal attention:
+        # few rows (at most the head count by length of every token) take the
+        # key-split tiles, which read the row count on the device
+        structured = fits and not (local_w >= T and L >= T and not use_quant
+                                   and _sa._causal_tiles(B * T * self._active_k(T), D))
         return {"L": L, "stride": stride, "local_w": local_w, "slots": slots, "K": K, "use_quant": use_quant,
-                "w_eff": w_eff, "structured": structured}
+                "w_eff": w_eff, "structured": structured, "fits": fits}
 
     def _fork_stream(self, device: torch.device) -> torch.cuda.Stream:
         """The forward's second stream on `device` (default priority)."""
