@@ -182,6 +182,17 @@ int pfa_proto_ema_update(const float* sums, int G, int C, float decay,
                          void* protos, void* usage, void* confidence,
                          int dtype, void* stream);
 
+/* The router's tail in two launches: pfa_proto_partial_reduce and
+ * pfa_proto_ema_update of the n_parts partials (none with n_parts = 0),
+ * pfa_router_stats_reduce of the n_blocks statistics (none with stats NULL)
+ * and heads64[i] = heads[i] for i < n_heads. */
+int pfa_router_tail(float* partial, int n_parts, int G, int C, float decay,
+                    float* sums, void* protos, void* usage, void* confidence,
+                    int dtype, const float* stats, int n_blocks,
+                    double* stats_out, const int32_t* heads, int n_heads,
+                    int64_t* heads64, void* stream);
+
+
 /* ====================================================================
  * Token top-k: per batch row keep the `need` highest importance tokens
  * (ties -> lowest index), need = clamp(max(keep_count, #(imp >= threshold),

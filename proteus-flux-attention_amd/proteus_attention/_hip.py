@@ -36,6 +36,7 @@ EXPORTED_SYMBOLS = (
     "pfa_router_raw_workspace_size",
     "pfa_router_topk_raw_ws",
     "pfa_proto_ema_update",
+    "pfa_router_tail",
     "pfa_proto_partial_count",
     "pfa_proto_accumulate",
     "pfa_proto_partial_reduce",
@@ -112,6 +113,8 @@ _SIGNATURES = {
     "pfa_router_topk_raw_ws": ([_vp, _i32, _i64, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i32,
                                 _f32, _f32, _f32, _f32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
                                _i32),
+    "pfa_router_tail": ([_vp, _i32, _i32, _i32, _f32, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _vp, _i32, _vp, _vp],
+                        _i32),
     "pfa_proto_ema_update": ([_vp, _i32, _i32, _f32, _vp, _vp, _vp, _i32, _vp], _i32),
     "pfa_proto_partial_count": ([_i64, ctypes.POINTER(_i32)], _i32),
     "pfa_proto_accumulate": ([_vp, _i32, _i64, _i32, _i32, _vp, _vp, _i32, _vp], _i32),

@@ -937,26 +937,32 @@ class AdaptiveSparseAttention(nn.Module):
         return bool(self.proto_enabled and self.routing_prototypes is not None
                     and self.routing_usage_ema is not None and self.routing_confidence is not None)
 
-    def _update_routing_prototypes(self, token_feats: torch.Tensor, gate_probs: torch.Tensor) -> None:
-        """Prototype / usage / confidence EMA (aspa.py:692-718)."""
-        if not self._ema_active():
-            return
-        with torch.no_grad():
-            lib = _hip.lib()
-            x2d = token_feats.detach().reshape(-1, self.d_model)
+    def _update_routing_prototypes(self, token_feats: torch.Tensor, gate_probs: torch.Tensor,
+                                   stats: Optional[torch.Tensor] = None, comb: Optional[torch.Tensor] = None,
+                                   heads: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+        """Prototype / usage / confidence EMA (aspa.py:692-718) and, in the same
+        launches (pfa_router_tail), the reduction of the router statistics
+        `stats` into the first 64 bytes of `comb` and the int64 copy of the
+        int32 head list `heads`, which is returned."""
+        lib = _hip.lib()
+        C, G = self.d_model, self.attn_gates
+        device = token_feats.device
+        partial = sums = None
+        nparts, protos = 0, (None, None, None, 0)
+        if self._ema_active():
+            x2d = token_feats.detach().reshape(-1, C)
             if x2d.dtype not in (torch.float32, torch.bfloat16, torch.float16):
                 x2d = x2d.to(torch.float32)
             x2d = x2d.contiguous()
-            device = x2d.device
-            n_tok, C, G = x2d.size(0), self.d_model, self.attn_gates
-            fused = getattr(self, "_ema_partial", None)
+            n_tok = x2d.size(0)
+            fused = self.__dict__.get("_ema_partial")
             self._ema_partial = None
             if fused is not None and fused[1] == x2d.data_ptr() and fused[2] == n_tok:
                 # statistics already accumulated by this forward's router pass
                 partial = fused[0]
                 nparts = partial.size(0)
             else:
-                probs = gate_probs.detach().to(torch.float32).reshape(-1, self.attn_gates).contiguous()
+                probs = gate_probs.detach().to(torch.float32).reshape(-1, G).contiguous()
                 np_c = _hip.ctypes.c_int(0)
                 _hip.check(lib.pfa_proto_partial_count(n_tok, _hip.ctypes.byref(np_c)), "pfa_proto_partial_count")
                 nparts = np_c.value
@@ -965,16 +971,21 @@ class AdaptiveSparseAttention(nn.Module):
                                                     _hip.ptr(probs), _hip.ptr(partial), nparts,
                                                     _hip.stream_ptr(device)), "pfa_proto_accumulate")
             sums = torch.empty(G, C + 1, dtype=torch.float32, device=device)
-            _hip.check(lib.pfa_proto_partial_reduce(_hip.ptr(partial), nparts, G, C, _hip.ptr(sums),
-                                                    _hip.stream_ptr(device)), "pfa_proto_partial_reduce")
             proto, usage, conf = self.routing_prototypes, self.routing_usage_ema, self.routing_confidence
             if not (proto.dtype == usage.dtype == conf.dtype and proto.is_contiguous()):
                 raise ValueError("routing_prototypes / routing_usage_ema / routing_confidence must share one "
                                  "dtype and be contiguous")
-            _hip.check(lib.pfa_proto_ema_update(_hip.ptr(sums), G, C, float(self.proto_decay), _hip.ptr(proto),
-                                                _hip.ptr(usage), _hip.ptr(conf), _hip.dtype_tag(proto.dtype),
-                                                _hip.stream_ptr(device)), "pfa_proto_ema_update")
+            protos = (_hip.ptr(proto), _hip.ptr(usage), _hip.ptr(conf), _hip.dtype_tag(proto.dtype))
+        elif stats is None and heads is None:
+            return None
+        heads64 = torch.empty(heads.numel(), dtype=torch.int64, device=device) if heads is not None else None
+        _hip.check(lib.pfa_router_tail(_hip.ptr(partial), nparts, G, C, float(self.proto_decay), _hip.ptr(sums), *protos,
+                                       _hip.ptr(stats), int(stats.size(0)) if stats is not None else 0, _hip.ptr(comb),
+                                       _hip.ptr(heads), int(heads.numel()) if heads is not None else 0,
+                                       _hip.ptr(heads64), _hip.stream_ptr(device)), "pfa_router_tail")
+        if sums is not None:
             self._proto_sums = sums
+        return heads64
 
     # ------------------------------------------------------------------
     def _full_rows(self, B: int, T: int, device: torch.device):
@@ -1413,12 +1424,9 @@ class AdaptiveSparseAttention(nn.Module):
         def ema() -> None:
             # the router's tail: the prototype EMA and the telemetry reduction
             # (both read only router outputs; neither is read in this forward)
-            self._update_routing_prototypes(x, gate_probs)
-            # the int64 active-head list of the sparse state, made here (off the
+            # the int64 active-head list of the sparse state is made here (off the
             # critical path) rather than when the telemetry is read
-            heads64[0] = active_heads.to(torch.int64)
-            _hip.check(lib.pfa_router_stats_reduce(_hip.ptr(router_stats), int(router_stats.size(0)), _hip.ptr(comb),
-                                                   _hip.stream_ptr(device)), "pfa_router_stats_reduce")
+            heads64[0] = self._update_routing_prototypes(x, gate_probs, router_stats, comb, active_heads)
         if sim is not None:
             self._last_token_similarity = sim.view(B, T)
             self._last_token_blend = blend.view(B, T)
