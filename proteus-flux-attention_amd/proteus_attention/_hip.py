@@ -209,7 +209,9 @@ def dtype_tag(dtype: torch.dtype) -> int:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    """The handle of torch's current stream on `device`."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -32,12 +32,14 @@ training-mode attention dropout.
 """
 from __future__ import annotations
 
+import contextlib
 import gc
 import math
 import time
 import warnings
 from typing import Any, Dict, Optional, Tuple
 
+import numpy as np
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
@@ -60,6 +62,20 @@ from ..kernels.sparse_attn import (
 # Every use is bracketed by stream waits in both directions, so sharing adds
 # no dependency a forward does not already have.
 _SIDE_STREAMS: Dict[Tuple[int, str], torch.cuda.Stream] = {}
+
+
+# An eager forward of fewer input elements (B * T * C) runs on the calling
+# stream alone.  The second stream lets the projection chain run beside the
+# router chain, but its fork, join and stream switches cost the host 60-100 us
+# a forward, more than the overlap gives while the host's launches bound it.
+# Measured on one box, one stream / two (us a call, C = 512, 8 heads x 64):
+#   bf16 shortlist, T = 1,024: 273 / 396; 16,384: 271 / 420; 40,960: 421 / 463;
+#     49,152: 482 / 425; 98,304: 711 / 663
+#   bf16 int8, 2 x 8,192: 370 / 476; 32,768: 428 / 504
+#   f32 shortlist, T = 4,096: 302 / 354; 6,000: 401 / 404; 10,007: 576 / 554
+#   f16 shortlist, T = 8,192: 336 / 408; 16,384: 516 / 510
+# f32 and f16 layers attend gathered candidates and keep the device longer.
+_ONE_STREAM_ELEMS = {torch.bfloat16: 21 << 20, torch.float16: 4 << 20, torch.float32: 3 << 20}
 
 
 def _side_stream(device: torch.device, role: str) -> torch.cuda.Stream:
@@ -560,27 +576,37 @@ class AdaptiveSparseAttention(nn.Module):
             keep += 1
         return min(max_cap, max(1, keep))
 
-    def _defer(self, fn) -> None:
-        """Queue a telemetry step that needs device results; it runs at the
-        next _resolve_stats (a telemetry read or the next forward) as
-        fn(module).  The steps take the module as their argument rather than
-        closing over it: a queued closure holding the module would make a
-        reference cycle, and a dropped module (with its device buffers and
-        graphs) would then live until Python's cycle collector ran."""
-        self.__dict__.setdefault("_pending_stats", []).append(fn)
+    def _defer(self, fn, build=None) -> None:
+        """Queue a telemetry step that needs device results: fn(module) reads
+        them and updates the running averages, build(module) fills the
+        dictionaries a reader sees.  Both run at the next _resolve_stats (a
+        telemetry read); the next forward runs fn alone and drops build, whose
+        dictionaries it replaces unread.  The steps take the module as their
+        argument rather than closing over it: a queued closure holding the
+        module would make a reference cycle, and a dropped module (with its
+        device buffers and graphs) would then live until Python's cycle
+        collector ran."""
+        self.__dict__.setdefault("_pending_stats", []).append((fn, build))
 
-    def _resolve_stats(self) -> None:
+    def _resolve_stats(self, build: bool = True) -> None:
         pend = self.__dict__.get("_pending_stats")
         if not pend:
             return
         self.__dict__["_pending_stats"] = []
-        for fn in pend:
-            fn(self)
+        for fn, _ in pend:
+            if fn is not None:
+                fn(self)
+        if build:
+            for _, fn in pend:
+                if fn is not None:
+                    fn(self)
 
     def _update_density(self, value: float) -> None:
         value = float(max(0.0, value))
-        self._last_density = value
-        self._density_ema = value if self._density_ema is None else 0.8 * self._density_ema + 0.2 * value
+        d = self.__dict__
+        ema = d.get("_lazy__density_ema")
+        d["_lazy__last_density"] = value
+        d["_lazy__density_ema"] = value if ema is None else 0.8 * ema + 0.2 * value
 
     def _density_threshold(self) -> Optional[float]:
         return self._dense_threshold
@@ -805,13 +831,13 @@ class AdaptiveSparseAttention(nn.Module):
                     raise ValueError("routing_prototypes / routing_confidence / routing_usage_ema must share one dtype")
         return w, protos, conf_b, usage_b, buf_dtype, use_proto
 
-    def _router_inputs(self, device: torch.device, x_dtype: torch.dtype):
+    def _router_inputs(self, device: torch.device, x_dtype: torch.dtype, raw=None):
         """Router weight table, prototype prior inputs (aspa.py:636-663) in one
         launch (pfa_router_prepare): (w_packed, conf_weight, usage_bias,
-        use_proto)."""
+        use_proto).  raw: _router_raw_inputs' result."""
         lib = _hip.lib()
         G, C = self.attn_gates, self.d_model
-        w, protos, conf_b, usage_b, buf_dtype, use_proto = self._router_raw_inputs(device)
+        w, protos, conf_b, usage_b, buf_dtype, use_proto = raw or self._router_raw_inputs(device)
         Gp = int(lib.pfa_router_gate_pad(G))
         wpk = torch.empty(C, 2 * Gp, dtype=torch.float32, device=device)
         conf = torch.empty(G, dtype=torch.float32, device=device) if conf_b is not None else None
@@ -843,7 +869,8 @@ class AdaptiveSparseAttention(nn.Module):
         G, H = self.attn_gates, self.h_total
         # bf16 shapes of the MFMA router build their inputs inside the router
         # (pfa_router_topk_raw); the others take pfa_router_prepare first
-        w, protos, conf_b, usage_b, buf_dtype, use_proto = self._router_raw_inputs(device)
+        inputs = self._router_raw_inputs(device)
+        w, protos, conf_b, usage_b, buf_dtype, use_proto = inputs
         raw = bool(lib.pfa_router_raw_supported(_hip.dtype_tag(x2d.dtype), _hip.dtype_tag(w.dtype),
                                                 _hip.dtype_tag(buf_dtype), G, C, 1 if use_proto else 0))
         if raw:
@@ -851,7 +878,7 @@ class AdaptiveSparseAttention(nn.Module):
             if keep is not None:
                 keep.extend(t for t in (w, protos, conf_b, usage_b) if t is not None)
         else:
-            wpk, conf, usage, use_proto = self._router_inputs(device, x2d.dtype)
+            wpk, conf, usage, use_proto = self._router_inputs(device, x2d.dtype, inputs)
         gate = torch.empty(n_tok, G, dtype=torch.float32, device=device)
         imp = torch.empty(n_tok, dtype=torch.float32, device=device)
         sim = torch.empty(n_tok, dtype=torch.float32, device=device) if use_proto else None
@@ -914,7 +941,7 @@ class AdaptiveSparseAttention(nn.Module):
             return mask
         guard = min(max(0, self.token_keep_guard), T)
         min_keep = max(min(max(0, self.token_keep_min), T), guard)
-        keep = int(torch.tensor(ratio * T, dtype=torch.float32).round().item())
+        keep = int(np.float32(ratio * T).round())  # half to even in f32, as torch rounds
         if min_keep > 0:
             keep = max(keep, min_keep)
         keep = max(1, min(keep, T))
@@ -1259,15 +1286,28 @@ class AdaptiveSparseAttention(nn.Module):
             self._capture_keep = []
             # no garbage collection inside the capture: a dead object that
             # owns device resources (pinned host memory, events) would be
-            # freed while the stream captures, which is not allowed; dead
-            # cycles are collected first
-            gc.collect()
+            # freed while the stream captures, which is not allowed.  With the
+            # collector off none starts, so dead cycles need no collection
+            # first (24 ms in a process with a torch heap).  The allocator's
+            # cache is kept where the card has as much free memory besides
+            # (torch.cuda.graph always empties it: 4 ms, and the buffers around
+            # the capture are then allocated from the driver again); a capture
+            # cannot release cached blocks itself.
             gc_was_on = gc.isenabled()
             gc.disable()
             try:
-                with torch.cuda.graph(graph, pool=self._hip_graph_pool):
-                    attn, stats_args, label = self._forward_impl(xs, capture=True)
-                    y_static = self.dropout(self.proj(attn)) if self._hip_graph_static_output else None
+                torch.cuda.synchronize(device)
+                cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+                if torch.cuda.mem_get_info(device)[0] < cached:
+                    torch.cuda.empty_cache()
+                side = _side_stream(device, "capture")
+                with torch.cuda.stream(side):
+                    graph.capture_begin(pool=self._hip_graph_pool)
+                    try:
+                        attn, stats_args, label = self._forward_impl(xs, capture=True)
+                        y_static = self.dropout(self.proj(attn)) if self._hip_graph_static_output else None
+                    finally:
+                        graph.capture_end()
             finally:
                 if gc_was_on:
                     gc.enable()
@@ -1316,18 +1356,23 @@ class AdaptiveSparseAttention(nn.Module):
             if not ended:
                 ev1.record()
 
-            def latency(self, st=st_now):
+            got = []
+
+            def latency(self):
                 ev1.synchronize()
                 ms = float(ev0.elapsed_time(ev1))
+                got.append(ms)
                 prev = self.__dict__.get("_lazy__latency_ema")
-                self._latency_ema = ms if prev is None else 0.8 * prev + 0.2 * ms
+                self.__dict__["_lazy__latency_ema"] = ms if prev is None else 0.8 * prev + 0.2 * ms
+
+            def latency_dicts(self, st=st_now):
                 hs = self.__dict__.get("_lazy_last_head_stats")
                 if hs is not None:
-                    hs["latency_ms"] = ms
+                    hs["latency_ms"] = got[0]
                 if st is not None:
-                    st["latency_ms"] = ms
+                    st["latency_ms"] = got[0]
 
-            self._defer(latency)
+            self._defer(latency, latency_dicts)
 
         def labels(self, st=st_now):
             hs = self.__dict__.get("_lazy_last_head_stats")
@@ -1337,7 +1382,7 @@ class AdaptiveSparseAttention(nn.Module):
             if st is not None:
                 st["mode_selected"] = label
 
-        self._defer(labels)
+        self._defer(None, labels)
 
     def _forward_impl(self, x: torch.Tensor, capture: bool = False):
         """The forward (aspa.py:1442-1932).  With capture=True nothing waits
@@ -1345,18 +1390,21 @@ class AdaptiveSparseAttention(nn.Module):
         left to the caller: returns (attn, stats_args, label)."""
         B, T, C = x.shape
         device = x.device
-        self.last_aux_loss = None
-        self._last_token_importance = None
-        self._last_token_mask = None
-        self._last_token_blend = None
+        # plain attributes are written into the instance dictionary: a Module's
+        # __setattr__ looks for parameters and submodules first (1 us each)
+        plain = self.__dict__
+        plain["last_aux_loss"] = None
+        plain["_last_token_importance"] = None
+        plain["_last_token_mask"] = None
+        plain["_last_token_blend"] = None
         if not self.proto_enabled:
-            self._last_token_similarity = None
+            plain["_last_token_similarity"] = None
         ev0 = ev1 = None
         if self.track_latency and not capture:
             ev0 = torch.cuda.Event(enable_timing=True)
             ev1 = torch.cuda.Event(enable_timing=True)
             ev0.record()
-        self._last_batch_size = B
+        plain["_last_batch_size"] = B
 
         def finish(label: str) -> None:
             self._finish_forward(label, ev0, ev1)
@@ -1370,19 +1418,23 @@ class AdaptiveSparseAttention(nn.Module):
         # anchor pass run on a forked stream while the router, packing, the
         # prototype EMA and the prototype prefix tables run on the calling
         # stream; the main attention pass joins them.
-        main_s = torch.cuda.current_stream(device)
-        fork_s = self._fork_stream(device)
-        fork_s.wait_stream(main_s)
-        with torch.cuda.stream(fork_s):
+        # (a small eager forward keeps to the calling stream: _ONE_STREAM_ELEMS)
+        one_stream = not capture and B * T * C < _ONE_STREAM_ELEMS.get(x.dtype, 0)
+        main_s = fork_s = None
+        if not one_stream:
+            main_s = torch.cuda.current_stream(device)
+            fork_s = self._fork_stream(device)
+            fork_s.wait_stream(main_s)
+        with contextlib.nullcontext() if one_stream else torch.cuda.stream(fork_s):
             qkv = self.qkv(x).contiguous()  # (B, T, 3C) = (B, T, 3, H, D)
 
         alpha = self._compute_cvt_alpha(T)
-        self._current_alpha = alpha
+        plain["_current_alpha"] = alpha
         if self.token_sparse:
             blend_ratio = (1.0 - alpha) * float(self.token_keep_ratio_base) + alpha * float(self._linear_token_keep_ratio(T))
-            self._token_keep_ratio_runtime = float(max(0.0, min(1.0, blend_ratio)))
+            plain["_token_keep_ratio_runtime"] = float(max(0.0, min(1.0, blend_ratio)))
         else:
-            self._token_keep_ratio_runtime = None
+            plain["_token_keep_ratio_runtime"] = None
 
         # head count (aspa.py:1574-1589); nucleus count needs head probs, so
         # the router is run with topk chosen after it when top_p > 0.
@@ -1407,14 +1459,14 @@ class AdaptiveSparseAttention(nn.Module):
         linear_topk = max(1, min(adaptive_topk, self.linear_head_k))
         topk = max(1, int(round((1.0 - alpha) * float(adaptive_topk) + alpha * float(linear_topk))))
         topk = min(adaptive_topk, topk)
-        self._last_target_k = topk
+        plain["_last_target_k"] = topk
         if topk == dense_topk:
             hidx, hsc = hidx_all, hsc_all
         else:
             hidx = hidx_all[:, :topk].contiguous()
             hsc = hsc_all[:, :topk].contiguous()
         gate_probs = gate.view(B, T, self.attn_gates)
-        self._last_gate_probs = gate_probs
+        plain["_last_gate_probs"] = gate_probs
         # the prototype EMA (aspa.py:692-718) reads only this forward's router
         # outputs and is read only by the next forward's router: it is queued
         # last before the streams join (on the structured path beside the
@@ -1428,16 +1480,16 @@ class AdaptiveSparseAttention(nn.Module):
             # critical path) rather than when the telemetry is read
             heads64[0] = self._update_routing_prototypes(x, gate_probs, router_stats, comb, active_heads)
         if sim is not None:
-            self._last_token_similarity = sim.view(B, T)
-            self._last_token_blend = blend.view(B, T)
+            plain["_last_token_similarity"] = sim.view(B, T)
+            plain["_last_token_blend"] = blend.view(B, T)
         else:
-            self._last_token_similarity = None
-            self._last_token_blend = None
-        self._last_proto_stats = None
+            plain["_last_token_similarity"] = None
+            plain["_last_token_blend"] = None
+        plain["_lazy__last_proto_stats"] = None
         importance = imp.view(B, T)
-        self._last_token_importance = importance
+        plain["_last_token_importance"] = importance
         token_mask = self._select_active_tokens(importance)
-        self._last_token_mask = token_mask
+        plain["_last_token_mask"] = token_mask
 
         router_reg = self._router_regulariser(gate_probs)
 
@@ -1496,7 +1548,7 @@ class AdaptiveSparseAttention(nn.Module):
             P, N, max_rows = -1, B * cap * topk, -1
         else:
             P, N, max_rows = -1, B * T * topk, -1
-        self._pending_summary = None if need_summary else summary
+        plain["_pending_summary"] = None if need_summary else summary
         density_est = float(max_rows) / float(max(1, T)) if max_rows >= 0 else 0.0
         all_rows_active = N == BH * T
         prefer_dense = alpha <= self.dense_alpha_cutoff and not self.quantize_sparse_int8
@@ -1525,7 +1577,7 @@ class AdaptiveSparseAttention(nn.Module):
         fuse = 0
         if q_fused and self.d_head == 64 and self.fuse_anchor_pass and plan["stride"] > 0 and plan["slots"] > 0:
             fuse = _sa.FUSE_ZERO | (_sa.FUSE_K_ROPE if (self.use_rope and self.fuse_k_rope) else 0)
-        with torch.cuda.stream(fork_s):
+        with contextlib.nullcontext() if one_stream else torch.cuda.stream(fork_s):
             rot_k = not (fuse & _sa.FUSE_K_ROPE)
             if fuse:
                 attn = torch.empty(B, T, C, dtype=qkv.dtype, device=device)
@@ -1537,21 +1589,22 @@ class AdaptiveSparseAttention(nn.Module):
             else:
                 q_rope = self._rope_inplace(qkv, rotate_q=not q_fused, rotate_k=rot_k)
                 attn = torch.zeros(B, T, C, dtype=qkv.dtype, device=device)
-        if not capture:
+        if not capture and not one_stream:
             # the forked stream's tensors are used (and freed) on this stream
             qkv.record_stream(main_s)
             attn.record_stream(main_s)
         # The structured path keeps the two streams apart up to the main pass;
         # the others (and the int8 mode, which quantises q/k/v first) join here.
-        join_early = not structured or use_quant
+        join_early = not structured or use_quant or one_stream
         if join_early:
             ema()
-            main_s.wait_stream(fork_s)
+            if not one_stream:
+                main_s.wait_stream(fork_s)
         D = self.d_head
         mode_label = "sparse"
         if force_dense:
-            self._cached_active_mask = None
-            self._cached_packing = None
+            plain["_cached_active_mask"] = None
+            plain["_cached_packing"] = None
             # a token mask keeps the rows of the kept tokens only; the others
             # stay zero (attn starts zeroed)
             self._attend_dense_causal(qkv, B, T, attn, token_mask=token_mask)
@@ -1560,7 +1613,7 @@ class AdaptiveSparseAttention(nn.Module):
             else:
                 mode_label = "dense_auto"  # refined to "dense" once P is read back
             _record_backend("hip_dense", device=str(device), heads=BH, tokens=T, max_rows=T, quantized=False)
-            self._last_sparse_state = {
+            plain["_lazy__last_sparse_state"] = {
                 "mode": mode_label, "backend": get_last_backend(), "max_rows": max_rows, "density": density_est,
                 "target_k": int(topk),
                 "force_dense_threshold": None if density_threshold is None else float(density_threshold),
@@ -1570,9 +1623,9 @@ class AdaptiveSparseAttention(nn.Module):
             }
         elif P == 0 or N == 0 or (not need_summary and B * T == 0):
             dense_reason = None
-            self._cached_active_mask = None
-            self._cached_packing = None
-            self._last_sparse_state = {
+            plain["_cached_active_mask"] = None
+            plain["_cached_packing"] = None
+            plain["_lazy__last_sparse_state"] = {
                 "mode": "dense", "backend": "not_invoked", "max_rows": max_rows, "density": density_est,
                 "target_k": int(topk),
                 "force_dense_threshold": None if density_threshold is None else float(density_threshold),
@@ -1608,9 +1661,9 @@ class AdaptiveSparseAttention(nn.Module):
             if isinstance(det, dict):
                 for key, val in det.items():
                     state[f"linear_shortlist_{key}"] = val
-            self._last_sparse_state = state
-        self.last_head_consensus = None if self.training else attn.detach()
-        self.last_router_reg = router_reg
+            plain["_lazy__last_sparse_state"] = state
+        plain["last_head_consensus"] = None if self.training else attn.detach()
+        plain["last_router_reg"] = router_reg
         stats_args = (token_mask, topk, adaptive_topk, P, N, max_rows, density_threshold, alpha, mode_label,
                       dense_reason, B, T, active_heads, row_offsets, summary, comb)
         label = f"cvt(alpha={alpha:.2f})::{mode_label}"
@@ -1855,23 +1908,20 @@ class AdaptiveSparseAttention(nn.Module):
         the next forward), so the forward never stalls the device queue.
         done: an event of the caller's, not yet recorded, that is recorded
         here after the copy (the caller's latency end event), or None."""
-        self._resolve_stats()
+        # the previous forward's values leave the staging tensor here
+        self._resolve_stats(build=False)
         H = self.h_total
-        with torch.no_grad():
-            # one pinned staging tensor, kept across forwards: the previous
-            # forward's values were consumed by _resolve_stats above
-            h = self.__dict__.get("_stats_host")
-            if h is None or h.shape != comb.shape:
-                h = torch.empty(comb.shape, dtype=torch.int32, pin_memory=True)
-                self.__dict__["_stats_host"] = h
-            h.copy_(comb, non_blocking=True)
-            host = (h[:16].view(torch.float64), h[16:20], h[20:])
+        d = self.__dict__
+        # one pinned staging tensor, kept across forwards
+        host = d.get("_stats_host")
+        if host is None or host.shape != comb.shape:
+            host = d["_stats_host"] = torch.empty(comb.shape, dtype=torch.int32, pin_memory=True)
+        host.copy_(comb, non_blocking=True)
+        if done is None:
+            done = d.get("_stats_event")
             if done is None:
-                done = self.__dict__.get("_stats_event")
-                if done is None:
-                    done = torch.cuda.Event()
-                    self.__dict__["_stats_event"] = done
-            done.record()
+                done = d["_stats_event"] = torch.cuda.Event()
+        done.record()
         # everything the dictionaries need from the host side, as of now
         st = self.__dict__.get("_lazy__last_sparse_state")
         info = self._last_shortlist_backend_info or get_last_backend_info()
@@ -1880,17 +1930,23 @@ class AdaptiveSparseAttention(nn.Module):
                                                            int(self.linear_anchor_stride)),
             proto=self._last_token_similarity is not None, mode_setting=self.mode_setting)
 
+        got: Dict[str, Any] = {}
+
+        def read(self) -> None:
+            done.synchronize()
+            words = host.numpy()
+            got["part"] = words[:16].view(np.float64).tolist()
+            got["summ"] = words[16:].tolist()
+            self._update_density(float(got["summ"][2]) / float(max(1, T)))
+
         def build(self) -> None:
             nonlocal mode_label
-            done.synchronize()
-            part = host[0].tolist()
-            summ = host[1].tolist()
-            ent_sum, sim_sum, blend_sum, blend_pos, score_sum = part[:5]
+            summ = got["summ"]
+            ent_sum, sim_sum, blend_sum, blend_pos, score_sum = got["part"][:5]
             P_, N_, max_rows_ = int(summ[0]), int(summ[1]), int(summ[2])
-            heads_list = host[2][:P_].tolist()
+            heads_list = summ[4:4 + P_]
             n_tok = max(1, B * T)
             density_est = float(max_rows_) / float(max(1, T))
-            self._update_density(density_est)
             keep_frac = float(N_) / float(max(1, topk * B * T)) if token_mask is not None else 1.0
             if mode_label == "dense_auto" and P_ == B * H:
                 mode_label = "dense"
@@ -1949,7 +2005,7 @@ class AdaptiveSparseAttention(nn.Module):
             self._last_proto_stats = proto_stats
             self.last_head_stats = hs
 
-        self._defer(build)
+        self._defer(read, build)
 
 
 class AdaptiveSparseProtoAttention(AdaptiveSparseAttention):
