@@ -99,12 +99,21 @@ struct ShortArgs {
   __device__ __forceinline__ float head_out_scale(int bh) const { return vsc ? vsc[bh] : 1.f; }
 };
 
-// NH: 64-dim halves of the head (1, or 2 for D = 128); acc[4 * NH] holds
-// the lane's output dims 16db + 4g .. +3.
-template <int NH>
+// The kernels' head width, as ND 16-dim output blocks: 1, 2, 4 or 8 for D =
+// 16, 32, 64 or 128.  A tile row holds 64 dims (two such halves for D = 128);
+// of a narrow row (D < 64) only the chunks a product reads are filled, one
+// 32-dim score product is taken and ND output blocks are kept.  At 65,536
+// tokens x 32 heads x 16 dims the passes that treated narrow rows as 64 wide
+// took 277 us (main) and 156 us (anchor); now 250 and 116 us, bound by the
+// softmax, whose work does not depend on D.
+constexpr int nd_halves(int ND) { return ND > 4 ? 2 : 1; }   // 64-dim halves of a tile row
+constexpr int nd_scores(int ND) { return ND > 2 ? ND / 2 : 1; }  // 32-dim score products
+
+// acc[ND] holds the lane's output dims 16db + 4g .. +3.
+template <int ND>
 struct QState {
   float m, l;
-  f32x4_t acc[4 * NH];
+  f32x4_t acc[ND];
   int cnt;
 };
 
@@ -269,8 +278,8 @@ __device__ __forceinline__ void window_qk(const bf16x8_t (&qf)[NQ], const Tile& 
 // the max rises) and returns P rounded to bf16 (v_cvt_pk_bf16_f32, round to
 // nearest even) as the two B operands of the P.V product, pb[kc] holding
 // keys 32kc + 4g + (0..3) and 32kc + 16 + 4g + (0..3).
-template <int NH>
-__device__ __forceinline__ void softmax_p(float (&s)[4][4], float scale_log2, QState<NH>& st, bf16x8_t (&pb)[2]) {
+template <int ND>
+__device__ __forceinline__ void softmax_p(float (&s)[4][4], float scale_log2, QState<ND>& st, bf16x8_t (&pb)[2]) {
   float tmax = -INFINITY;
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb)
@@ -287,7 +296,7 @@ __device__ __forceinline__ void softmax_p(float (&s)[4][4], float scale_log2, QS
     const float alpha = (mn == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(st.m - mn);  // st.m == -inf -> 0
     st.l *= alpha;
 #pragma unroll
-    for (int db = 0; db < 4 * NH; ++db)
+    for (int db = 0; db < ND; ++db)
 #pragma unroll
       for (int i = 0; i < 4; ++i) st.acc[db][i] *= alpha;
     st.m = mn;
@@ -336,28 +345,29 @@ __device__ __forceinline__ bf16x8_t v_frag(const Tile& t, int kc, int db) {
 // P.V products.
 // With two 64-dim halves the second half's V^T reads follow the first
 // half's products (the registers of one half's operands at a time).
-template <int NH, typename Tile>
-__device__ __forceinline__ void softmax_pv(float (&s)[4][4], const Tile& t, float scale_log2, QState<NH>& st) {
-  bf16x8_t va[2][4];
+template <int ND, typename Tile>
+__device__ __forceinline__ void softmax_pv(float (&s)[4][4], const Tile& t, float scale_log2, QState<ND>& st) {
+  constexpr int NB = ND < 4 ? ND : 4;  // output blocks of a half
+  bf16x8_t va[2][NB];
 #pragma unroll
   for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-    for (int db = 0; db < 4; ++db) va[kc][db] = v_frag(t, kc, db);
+    for (int db = 0; db < NB; ++db) va[kc][db] = v_frag(t, kc, db);
   bf16x8_t pb[2];
   softmax_p(s, scale_log2, st, pb);
 #pragma unroll
-  for (int h = 0; h < NH; ++h) {
+  for (int h = 0; h < nd_halves(ND); ++h) {
     if (h > 0) {
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-        for (int db = 0; db < 4; ++db) va[kc][db] = v_frag(t, kc, 4 * h + db);
+        for (int db = 0; db < NB; ++db) va[kc][db] = v_frag(t, kc, 4 * h + db);
     }
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
+      for (int db = 0; db < NB; ++db)
         st.acc[4 * h + db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[kc][db], pb[kc], st.acc[4 * h + db], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
   }
@@ -382,12 +392,12 @@ __device__ __forceinline__ void load_q(const uint16_t* qrow, bf16x8_t (&qf)[NQ],
 // would hold.
 // NARROW: chunks past cmask (a row of 16 or 32 dims, tables of that width)
 // are zero.
-template <bool NARROW>
+template <int NQ, bool NARROW>
 __device__ __forceinline__ void load_q_rope(const uint16_t* qrow, const uint16_t* crow, const uint16_t* srow,
-                                            bf16x8_t (&qf)[2], uint32_t cmask) {
+                                            bf16x8_t (&qf)[NQ], uint32_t cmask) {
   const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
-  for (int dc = 0; dc < 2; ++dc) {
+  for (int dc = 0; dc < NQ; ++dc) {
     if (NARROW && (uint32_t)(4 * dc + g) > cmask) {
       qf[dc] = bf16x8_t{};
       continue;
@@ -406,14 +416,14 @@ __device__ __forceinline__ void load_q_rope(const uint16_t* qrow, const uint16_t
 }
 
 // NARROW: a row of 16 or 32 dims (a.cmask); otherwise 32 * NQ dims.  The
-// RoPE tables on load are (T, D) for rows of at most 64 dims (NQ = 2,
+// RoPE tables on load are (T, D) for rows of at most 64 dims (NQ <= 2,
 // checked by the host).
 template <int NQ, bool NARROW>
 __device__ __forceinline__ void load_q_row(const ShortArgs& a, const uint16_t* qb, int64_t t, bf16x8_t (&qf)[NQ]) {
-  if constexpr (NQ == 2) {
+  if constexpr (NQ <= 2) {
     if (a.rcos != nullptr) {
       const int64_t tw = NARROW ? (int64_t)a.dh : 64;  // table row width
-      load_q_rope<NARROW>(qb + t * a.q.s_t, a.rcos + t * tw, a.rsin + t * tw, qf, NARROW ? a.cmask : 7u);
+      load_q_rope<NQ, NARROW>(qb + t * a.q.s_t, a.rcos + t * tw, a.rsin + t * tw, qf, NARROW ? a.cmask : 7u);
       return;
     }
   }
@@ -423,43 +433,53 @@ __device__ __forceinline__ void load_q_row(const ShortArgs& a, const uint16_t* q
 // dma_tile from wave-uniform K/V bases with 32-bit byte offsets per lane
 // (the caller checks that every offset of the sequence fits in 32 bits):
 // no 64-bit address arithmetic per tile.
-// NH = 2: the second 64-dim half of each row (source + 128 bytes) fills
-// the second K and V tiles of the stage (SwzTileH's layout).
-template <int NH>
+// D = 128: the second 64-dim half of each row (source + 128 bytes) fills
+// the second K and V tiles of the stage (SwzTileH's layout).  D < 64: only
+// the lanes whose chunk a product reads take part (the four chunks of the
+// score product, the 2 ND chunks of the output blocks).
+template <int ND>
 __device__ __forceinline__ void dma_tile32(const uint16_t* kb, const uint16_t* vb, uint32_t ks_t, uint32_t vs_t,
                                            int key0, int key1, uint32_t lds_w, uint32_t cmask) {
+  constexpr int NH = nd_halves(ND);
   const int tid = threadIdx.x;
-  const uint32_t c = 2u * 8u * ((uint32_t)((tid & 7) ^ tile_swz(tid >> 3)) & cmask);
+  const uint32_t lc = (uint32_t)((tid & 7) ^ tile_swz(tid >> 3));  // the slot's logical chunk
+  const uint32_t c = 2u * 8u * (lc & cmask);
   const uint32_t k2 = 2u * ks_t, v2 = 2u * vs_t;
   constexpr uint32_t kT = 2 * kSwzTileElems;  // bytes of one 64 x 64 tile
+  if (ND >= 4 || lc < 4) {
 #pragma unroll
-  for (int h = 0; h < NH; ++h) {
-    lds_dma16_s(kb, (uint32_t)key0 * k2 + c + 128u * h, lds_w + kT * h);
-    lds_dma16_s(kb, (uint32_t)key1 * k2 + c + 128u * h, lds_w + kT * h + 4096);
+    for (int h = 0; h < NH; ++h) {
+      lds_dma16_s(kb, (uint32_t)key0 * k2 + c + 128u * h, lds_w + kT * h);
+      lds_dma16_s(kb, (uint32_t)key1 * k2 + c + 128u * h, lds_w + kT * h + 4096);
+    }
   }
+  if (ND >= 4 || lc < 2 * ND) {
 #pragma unroll
-  for (int h = 0; h < NH; ++h) {
-    lds_dma16_s(vb, (uint32_t)key0 * v2 + c + 128u * h, lds_w + kT * (NH + h));
-    lds_dma16_s(vb, (uint32_t)key1 * v2 + c + 128u * h, lds_w + kT * (NH + h) + 4096);
+    for (int h = 0; h < NH; ++h) {
+      lds_dma16_s(vb, (uint32_t)key0 * v2 + c + 128u * h, lds_w + kT * (NH + h));
+      lds_dma16_s(vb, (uint32_t)key1 * v2 + c + 128u * h, lds_w + kT * (NH + h) + 4096);
+    }
   }
 }
-// dma_tile (64-bit addresses) for NH halves.
-template <int NH>
+// The same with 64-bit addresses.
+template <int ND>
 __device__ __forceinline__ void dma_tile_h(const uint16_t* kb, const uint16_t* vb, uint32_t ks_t, uint32_t vs_t,
                                            int key0, int key1, uint32_t lds_w, uint32_t cmask) {
+  constexpr int NH = nd_halves(ND);
   constexpr uint32_t kT = 2 * kSwzTileElems;
-  if constexpr (NH == 1) {
-    dma_tile(kb, vb, ks_t, vs_t, key0, key1, lds_w, cmask);
-  } else {
-    const int tid = threadIdx.x;
-    const int c = 8 * (int)((uint32_t)((tid & 7) ^ tile_swz(tid >> 3)) & cmask);
-    const uint64_t k0 = (uint64_t)(uint32_t)key0 * ks_t, k1 = (uint64_t)(uint32_t)key1 * ks_t;
-    const uint64_t v0 = (uint64_t)(uint32_t)key0 * vs_t, v1 = (uint64_t)(uint32_t)key1 * vs_t;
+  const int tid = threadIdx.x;
+  const uint32_t lc = (uint32_t)((tid & 7) ^ tile_swz(tid >> 3));
+  const int c = 8 * (int)(lc & cmask);
+  const uint64_t k0 = (uint64_t)(uint32_t)key0 * ks_t, k1 = (uint64_t)(uint32_t)key1 * ks_t;
+  const uint64_t v0 = (uint64_t)(uint32_t)key0 * vs_t, v1 = (uint64_t)(uint32_t)key1 * vs_t;
+  if (ND >= 4 || lc < 4) {
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
       lds_dma16(kb + c + 64 * h + k0, lds_w + kT * h);
       lds_dma16(kb + c + 64 * h + k1, lds_w + kT * h + 4096);
     }
+  }
+  if (ND >= 4 || lc < 2 * ND) {
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
       lds_dma16(vb + c + 64 * h + v0, lds_w + kT * (NH + h));
@@ -468,13 +488,13 @@ __device__ __forceinline__ void dma_tile_h(const uint16_t* kb, const uint16_t* v
   }
 }
 
-template <int NH>
-__device__ __forceinline__ void init_state(QState<NH>& st) {
+template <int ND>
+__device__ __forceinline__ void init_state(QState<ND>& st) {
   st.m = -INFINITY;
   st.l = 0.f;
   st.cnt = 0;
 #pragma unroll
-  for (int db = 0; db < 4 * NH; ++db) st.acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int db = 0; db < ND; ++db) st.acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 }
 
 __device__ __forceinline__ int64_t xcd_block(int64_t P, int64_t nblk) {
@@ -557,11 +577,12 @@ constexpr int kAnchorStages = 2;
 // residue classes, whose chunks each stream long key bands: the tile
 // transfers and barriers are then shared by twice the rows.
 constexpr int kAnchorNG2Positions = 256;  // class positions from which NG = 2 is launched
-// NARROW: rows of D = 16 or 32 elements (a.cmask); otherwise D = 64 * NH.
 // cm masks the tile DMA's chunk within a 64-dim half.
-template <int NG, bool NARROW, int NH>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NH == 1 ? 3 : 2, 8)))
+template <int NG, int ND>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ND <= 4 ? 3 : 2, 8)))
 short_anchor_kernel(ShortArgs a, int ccap) {
+  constexpr bool NARROW = ND < 4;
+  constexpr int NH = nd_halves(ND), NQ = nd_scores(ND);
   const uint32_t cm = NARROW ? a.cmask : 7u;
   constexpr int PW = part_w(NH);
   constexpr int S = kAnchorStages;
@@ -695,24 +716,24 @@ short_anchor_kernel(ShortArgs a, int ccap) {
       const int m0 = (int)mlo + kTile * i;
       const int ka = c + s * min(m0 + drow, (int)mhi), kz = c + s * min(m0 + drow + 32, (int)mhi);
       if (a.off32)
-        dma_tile32<NH>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz,
+        dma_tile32<ND>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz,
                        ring_w + kStageBytes * (uint32_t)(i % S), cm);
       else
-        dma_tile_h<NH>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz,
+        dma_tile_h<ND>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz,
                        ring_w + kStageBytes * (uint32_t)(i % S), cm);
     };
 #pragma unroll
     for (int i = 0; i < S - 1; ++i)
       if (i < ntile) request(i);
-    bf16x8_t qf[NG][2 * NH];
+    bf16x8_t qf[NG][NQ];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      load_q_row<2 * NH, NARROW>(a, qb, tq[g], qf[g]);
+      load_q_row<NQ, NARROW>(a, qb, tq[g], qf[g]);
 #pragma unroll
-      for (int dc = 0; dc < 2 * NH; ++dc)
+      for (int dc = 0; dc < NQ; ++dc)
         asm volatile("" : "+v"(qf[g][dc]));  // no load left for the tile loop to wait on
     }
-    QState<NH> st[NG];
+    QState<ND> st[NG];
 #pragma unroll
     for (int g = 0; g < NG; ++g) init_state(st[g]);
     for (int i = 0; i < ntile; ++i) {
@@ -749,7 +770,7 @@ short_anchor_kernel(ShortArgs a, int ccap) {
         const int gq = lane >> 4;
         if (gq == 0) { pr[0] = st[g].m; pr[1] = lt; }
 #pragma unroll
-        for (int db = 0; db < 4 * NH; ++db)
+        for (int db = 0; db < ND; ++db)
           *reinterpret_cast<f32x4_t*>(pr + 4 + 16 * db + 4 * gq) = st[g].acc[db];
       }
     }
@@ -788,11 +809,12 @@ struct MainOcc<3> {
   static constexpr int kWaves = 3;
 };
 
-// NARROW: rows of D = 16 or 32 elements; otherwise D = 64 * NH (cm as in
-// the anchor pass).
-template <bool COUNT, int S, bool NARROW, int NH>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NH == 1 ? MainOcc<S>::kWaves : 2, 8)))
+// (cm as in the anchor pass)
+template <bool COUNT, int S, int ND>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ND <= 4 ? MainOcc<S>::kWaves : 2, 8)))
 short_main_kernel(ShortArgs a, int use_part, int pcap) {
+  constexpr bool NARROW = ND < 4;
+  constexpr int NH = nd_halves(ND), NQ = nd_scores(ND);
   const uint32_t cm = NARROW ? a.cmask : 7u;
   constexpr int PW = part_w(NH);
   constexpr int kSlots = 16;  // tile slots of the shared window-tile schedule
@@ -889,9 +911,9 @@ short_main_kernel(ShortArgs a, int use_part, int pcap) {
     {
       const int ka = min(kTile * k_slot0 + drow, t_last), kz = min(kTile * k_slot0 + drow + 32, t_last);
       if (a.off32)
-        dma_tile32<NH>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz, ring_w, cm);
+        dma_tile32<ND>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz, ring_w, cm);
       else
-        dma_tile_h<NH>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz, ring_w, cm);
+        dma_tile_h<ND>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz, ring_w, cm);
     }
     const bool qv = qs >= s0 && qs < s1;
     const int tq = qv ? r_t[qs] : t_first;
@@ -1032,23 +1054,23 @@ short_main_kernel(ShortArgs a, int use_part, int pcap) {
     auto request = [&](int i) {
       const int ka = key_of(i, drow), kz = key_of(i, drow + 32);
       if (a.off32)
-        dma_tile32<NH>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz,
+        dma_tile32<ND>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz,
                        ring_w + kStageBytes * (uint32_t)(i % S), cm);
       else
-        dma_tile_h<NH>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz,
+        dma_tile_h<ND>(kb, vb, (uint32_t)a.k.s_t, (uint32_t)a.v.s_t, ka, kz,
                        ring_w + kStageBytes * (uint32_t)(i % S), cm);
     };
     if (!early) request(0);
 #pragma unroll
     for (int i = 1; i < S - 1; ++i)
       if (i < ntile) request(i);
-    bf16x8_t qf[2 * NH];
-    load_q_row<2 * NH, NARROW>(a, qb, tq, qf);
+    bf16x8_t qf[NQ];
+    load_q_row<NQ, NARROW>(a, qb, tq, qf);
     // settle the q fragments here: the tile loop then holds no load the
     // compiler would wait for (its wait would also drain the tile requests)
 #pragma unroll
-    for (int dc = 0; dc < 2 * NH; ++dc) asm volatile("" : "+v"(qf[dc]));
-    QState<NH> st;
+    for (int dc = 0; dc < NQ; ++dc) asm volatile("" : "+v"(qf[dc]));
+    QState<ND> st;
     init_state(st);
 
     // the rows of this wave are ascending in token: their key ranges lie in
@@ -1129,15 +1151,15 @@ short_main_kernel(ShortArgs a, int use_part, int pcap) {
       const int64_t r = r0 + qs;
       float m = st.m;
       float fa = 1.f, fb = 0.f, lp = 0.f;
-      f32x4_t pacc[4 * NH];
+      f32x4_t pacc[ND];
 #pragma unroll
-      for (int db = 0; db < 4 * NH; ++db) pacc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int db = 0; db < ND; ++db) pacc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       if (use_part) {
         const float* pr = a.part + r * PW;
         const float ma = pr[0];
         lp = pr[1];
 #pragma unroll
-        for (int db = 0; db < 4 * NH; ++db) pacc[db] = *reinterpret_cast<const f32x4_t*>(pr + 4 + 16 * db + 4 * g);
+        for (int db = 0; db < ND; ++db) pacc[db] = *reinterpret_cast<const f32x4_t*>(pr + 4 + 16 * db + 4 * g);
         const float mm = fmaxf(m, ma);
         fa = (m == -INFINITY) ? 0.f : exp2f(m - mm);
         fb = (ma == -INFINITY) ? 0.f : exp2f(ma - mm);
@@ -1146,8 +1168,7 @@ short_main_kernel(ShortArgs a, int use_part, int pcap) {
       const float inv = a.head_out_scale(bh) / den;
       uint16_t* op = (uint16_t*)a.out.ptr + bb * a.out.s_b + hh * a.out.s_h + (int64_t)tq * a.out.s_t;
 #pragma unroll
-      for (int db = 0; db < 4 * NH; ++db) {
-        if (NARROW && 16 * db + 4 * g >= a.dh) break;  // dims past D
+      for (int db = 0; db < ND; ++db) {
         uint16_t o4[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) o4[i] = f32_to_bf16((st.acc[db][i] * fa + pacc[db][i] * fb) * inv);
@@ -1254,13 +1275,18 @@ static int shortlist_attn_run(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, pfa_t
     const bool ng2 = npos >= kAnchorNG2Positions;
     if (D == 128) {
       // one row group per wave: two groups of 128-dim rows exceed the registers
-      short_anchor_kernel<1, false, 2><<<grid, 256, lds, s>>>(a, ccap);
+      short_anchor_kernel<1, 8><<<grid, 256, lds, s>>>(a, ccap);
     } else if (D == 64) {
-      if (ng2) short_anchor_kernel<2, false, 1><<<grid, 256, lds, s>>>(a, ccap);
-      else short_anchor_kernel<1, false, 1><<<grid, 256, lds, s>>>(a, ccap);
+      if (ng2) short_anchor_kernel<2, 4><<<grid, 256, lds, s>>>(a, ccap);
+      else short_anchor_kernel<1, 4><<<grid, 256, lds, s>>>(a, ccap);
     } else {
-      if (ng2) short_anchor_kernel<2, true, 1><<<grid, 256, lds, s>>>(a, ccap);
-      else short_anchor_kernel<1, true, 1><<<grid, 256, lds, s>>>(a, ccap);
+      if (D == 16) {
+        if (ng2) short_anchor_kernel<2, 1><<<grid, 256, lds, s>>>(a, ccap);
+        else short_anchor_kernel<1, 1><<<grid, 256, lds, s>>>(a, ccap);
+      } else {
+        if (ng2) short_anchor_kernel<2, 2><<<grid, 256, lds, s>>>(a, ccap);
+        else short_anchor_kernel<1, 2><<<grid, 256, lds, s>>>(a, ccap);
+      }
     }
     PFA_CHECK_LAUNCH("pfa_shortlist_attn_fwd/anchors");
   }
@@ -1280,14 +1306,19 @@ static int shortlist_attn_run(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, pfa_t
   const size_t dyn = (size_t)pcap * 12 + (size_t)ordcap * 4;
   const int up = anchors ? 1 : 0;
   if (D == 128) {
-    if (lengths != nullptr) short_main_kernel<true, S, false, 2><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
-    else short_main_kernel<false, S, false, 2><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+    if (lengths != nullptr) short_main_kernel<true, S, 8><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+    else short_main_kernel<false, S, 8><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
   } else if (D == 64) {
-    if (lengths != nullptr) short_main_kernel<true, S, false, 1><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
-    else short_main_kernel<false, S, false, 1><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+    if (lengths != nullptr) short_main_kernel<true, S, 4><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+    else short_main_kernel<false, S, 4><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
   } else {
-    if (lengths != nullptr) short_main_kernel<true, S, true, 1><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
-    else short_main_kernel<false, S, true, 1><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+    if (D == 16) {
+      if (lengths != nullptr) short_main_kernel<true, S, 1><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+      else short_main_kernel<false, S, 1><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+    } else {
+      if (lengths != nullptr) short_main_kernel<true, S, 2><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+      else short_main_kernel<false, S, 2><<<(unsigned)blocks, 256, dyn, s>>>(a, up, pcap);
+    }
   }
   PFA_CHECK_LAUNCH("pfa_shortlist_attn_fwd/main");
   return PFA_OK;
