@@ -364,6 +364,20 @@ int pfa_sparse_attn_fwd(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v,
                         float scale, const float* q_scale, const float* k_scale,
                         const float* v_scale, void* stream);
 
+/* pfa_sparse_attn_fwd with a workspace of (N + 15) / 16 bytes (NULL for none),
+ * which lets candidate rows share the keys of sixteen neighbours' lists. */
+int pfa_sparse_attn_fwd_ws(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v,
+                        int in_dtype, pfa_tensor4 out, int out_dtype, int H,
+                        int64_t T, int D, const int32_t* token_idx,
+                        const int32_t* row_head, const int32_t* head_map,
+                        int64_t N, const int32_t* n_rows_dev,
+                        const int32_t* cand, int64_t cand_stride,
+                        const int32_t* cand_len, const void* mask,
+                        int mask_dtype, const int32_t* head_max_token,
+                        float scale, const float* q_scale, const float* k_scale,
+                        const float* v_scale, void* workspace, size_t ws_bytes,
+                        void* stream);
+
 /* ====================================================================
  * Shortlist attention without materialised candidates (bf16, D = 16, 32,
  * 64 or 128; q_rope_cos / q_rope_sin need D <= 64 and the fused variant's

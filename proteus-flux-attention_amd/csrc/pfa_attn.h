@@ -39,6 +39,9 @@ struct AttnArgs {
   const float* k_scale;
   const float* v_scale;
   int mode;
+  // candidate rows: one byte per sixteen rows (the union kernel's verdict: 1
+  // where the row kernel is to attend them), or null
+  uint8_t* flags;
 };
 
 // Rows to process: the launch size, bounded by the device row count when one
@@ -153,5 +156,10 @@ int tile_attn_launch_f32(const AttnArgs& a, int out_dtype, int D, hipStream_t s)
 int tile_attn_launch_f16(const AttnArgs& a, int out_dtype, int D, hipStream_t s);
 int tile_attn_launch_bf16(const AttnArgs& a, int out_dtype, int D, hipStream_t s);
 int tile_attn_launch_i8(const AttnArgs& a, int out_dtype, int D, hipStream_t s);
+// The candidate kernel (pfa_cand_attn_<type>.hip), candidate rows without a mask.
+int cand_attn_launch_f32(const AttnArgs& a, int out_dtype, int D, hipStream_t s);
+int cand_attn_launch_f16(const AttnArgs& a, int out_dtype, int D, hipStream_t s);
+int cand_attn_launch_bf16(const AttnArgs& a, int out_dtype, int D, hipStream_t s);
+int cand_attn_launch_i8(const AttnArgs& a, int out_dtype, int D, hipStream_t s);
 
 }  // namespace pfa

@@ -25,7 +25,7 @@ sparse_attn_row_kernel(AttnArgs a) {
   using OT = typename Elem<ODT>::T;
   const int64_t lb = remap_block(blockIdx.x, gridDim.x);
   const int64_t r = lb * kAttnWaves + (threadIdx.x >> 6);
-  if (r >= attn_rows(a)) return;
+  if (r >= attn_rows(a) || (a.flags != nullptr && a.flags[r >> 4] == 0)) return;
 
   const int64_t t = a.token_idx[r];
   const int hp = a.row_head[r];
@@ -125,8 +125,24 @@ sparse_attn_generic_kernel(AttnArgs a, int D) {
   for (int dd = lane; dd < D; dd += 64) store_f<ODT>(op + dd, (l == 0.f) ? __builtin_nanf("") : accs[dd] / l);
 }
 
+// Candidate rows on the union kernel: where its fixed cost (about 20 us: marking
+// and listing a workgroup's keys) is covered by the candidates (at most N * L),
+// the table's ranges are few and the rows of a head lie close (on average, of
+// one batch row): lists of distant rows share little.  Measured (us, rows /
+// union):
+//   T = 8,192, spacing 4, 16,400 rows: bf16 134 / 55, f32 143 / 86; spacing 1,
+//     65,500 rows: 449 / 162, 514 / 267
+//   T = 4,096, spacing 4, 8,200 rows: bf16 55 / 36, f32 66 / 42
+//   T = 32,768, spacing 4, 65,700 rows: bf16 515 / 298, f32 723 / 581
+//   T = 65,536, spacing 80, 6,600 rows: bf16 49 / 54, f32 73 / 99
+//   T = 20,000, spacing 33, 4,800 rows: bf16 50 / 83, f32 82 / 131
+//   T = 1,024, 2,100 rows: bf16 12 / 21, f32 11 / 22
+constexpr int64_t kUnionEntries = 3 << 20;
+constexpr int64_t kUnionKeys = 32768;
+constexpr int64_t kUnionSpacing = 16;
+
 template <int IDT, int ODT>
-static int launch_attn(const AttnArgs& a, int D, hipStream_t s) {
+static int launch_attn(AttnArgs a, int D, hipStream_t s) {
   bool vec = (D % 8 == 0) && (D == 16 || D == 32 || D == 64 || D == 128);
   auto al = [](const pfa_tensor4& x, int esz) {
     return ((uintptr_t)x.ptr % (8 * esz)) == 0 && x.s_b % 8 == 0 && x.s_h % 8 == 0 && x.s_t % 8 == 0;
@@ -134,14 +150,28 @@ static int launch_attn(const AttnArgs& a, int D, hipStream_t s) {
   int ies = (IDT == PFA_F32) ? 4 : (IDT == PFA_I8 ? 1 : 2);
   int oes = (ODT == PFA_F32) ? 4 : 2;
   vec = vec && al(a.q, ies) && al(a.k, ies) && al(a.v, ies) && al(a.out, oes);
-  // Causal and masked rows of one head share their keys: tiles on the matrix
-  // cores.  Candidate rows each have their own keys, and bf16 inputs with
-  // f32 results would need P at more than the tiles' 16 bits: rows.
-  if (vec && a.mode != kModeCand && (a.mode != kModeMasked || a.T >= 4) && a.T < INT32_MAX / 2 && !(IDT == PFA_BF16 && ODT == PFA_F32)) {
-    if constexpr (IDT == PFA_F32) return tile_attn_launch_f32(a, ODT, D, s);
-    else if constexpr (IDT == PFA_F16) return tile_attn_launch_f16(a, ODT, D, s);
-    else if constexpr (IDT == PFA_BF16) return tile_attn_launch_bf16(a, ODT, D, s);
-    else return tile_attn_launch_i8(a, ODT, D, s);
+  // Rows of one head share keys: causal and masked rows on tiles of them,
+  // candidate rows on the union of sixteen lists, both on the matrix cores.
+  // bf16 inputs with f32 results would need P at more than the 16 bits those
+  // keep: rows, as for a mask beside candidates.  The row kernel behind the
+  // union kernel takes the rows it leaves.
+  if (vec && a.T < INT32_MAX / 2 && !(IDT == PFA_BF16 && ODT == PFA_F32)) {
+    if (a.mode != kModeCand && (a.mode != kModeMasked || a.T >= 4)) {
+      if constexpr (IDT == PFA_F32) return tile_attn_launch_f32(a, ODT, D, s);
+      else if constexpr (IDT == PFA_F16) return tile_attn_launch_f16(a, ODT, D, s);
+      else if constexpr (IDT == PFA_BF16) return tile_attn_launch_bf16(a, ODT, D, s);
+      else return tile_attn_launch_i8(a, ODT, D, s);
+    }
+    if (a.flags != nullptr) {
+      int rc;
+      if constexpr (IDT == PFA_F32) rc = cand_attn_launch_f32(a, ODT, D, s);
+      else if constexpr (IDT == PFA_F16) rc = cand_attn_launch_f16(a, ODT, D, s);
+      else if constexpr (IDT == PFA_BF16) rc = cand_attn_launch_bf16(a, ODT, D, s);
+      else rc = cand_attn_launch_i8(a, ODT, D, s);
+      if (rc != PFA_OK) return rc;
+    }
+  } else {
+    a.flags = nullptr;
   }
   if (vec) {
     int64_t blocks = (a.N + kAttnWaves - 1) / kAttnWaves;
@@ -166,13 +196,13 @@ static int launch_attn(const AttnArgs& a, int D, hipStream_t s) {
 
 using namespace pfa;
 
-extern "C" int pfa_sparse_attn_fwd(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, int in_dtype, pfa_tensor4 out,
+static int sparse_attn_run(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, int in_dtype, pfa_tensor4 out,
                                    int out_dtype, int H, int64_t T, int D, const int32_t* token_idx,
                                    const int32_t* row_head, const int32_t* head_map, int64_t N,
                                    const int32_t* n_rows_dev, const int32_t* cand,
                                    int64_t cand_stride, const int32_t* cand_len, const void* mask, int mask_dtype,
                                    const int32_t* head_max_token, float scale, const float* q_scale,
-                                   const float* k_scale, const float* v_scale, void* stream) {
+                                   const float* k_scale, const float* v_scale, uint8_t* flags, void* stream) {
   clear_error();
   PFA_CHECK_ARG(H > 0 && T > 0 && D > 0 && N >= 0, "pfa_sparse_attn_fwd: bad sizes H=%d T=%lld D=%d N=%lld", H,
                 (long long)T, D, (long long)N);
@@ -191,6 +221,8 @@ extern "C" int pfa_sparse_attn_fwd(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, 
   a.cand = cand; a.cand_stride = cand_stride; a.cand_len = cand_len; a.mask = mask; a.mask_dtype = mask_dtype;
   a.head_max = head_max_token; a.scale = scale; a.q_scale = q_scale; a.k_scale = k_scale; a.v_scale = v_scale;
   a.mode = cand ? kModeCand : (mask ? kModeMasked : kModeCausal);
+  a.flags = cand && !mask && N * cand_stride >= kUnionEntries && T <= kUnionKeys && T * H <= kUnionSpacing * N ? flags
+                                                                                                             : nullptr;
   hipStream_t s = as_stream(stream);
   if (in_dtype == PFA_F32 && out_dtype == PFA_F32) return launch_attn<PFA_F32, PFA_F32>(a, D, s);
   if (in_dtype == PFA_BF16 && out_dtype == PFA_BF16) return launch_attn<PFA_BF16, PFA_BF16>(a, D, s);
@@ -201,4 +233,34 @@ extern "C" int pfa_sparse_attn_fwd(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, 
   if (in_dtype == PFA_I8 && out_dtype == PFA_F16) return launch_attn<PFA_I8, PFA_F16>(a, D, s);
   set_error("pfa_sparse_attn_fwd: unsupported dtype pair in=%d out=%d", in_dtype, out_dtype);
   return PFA_E_UNSUPPORTED;
+}
+
+extern "C" int pfa_sparse_attn_fwd(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, int in_dtype, pfa_tensor4 out,
+                                   int out_dtype, int H, int64_t T, int D, const int32_t* token_idx,
+                                   const int32_t* row_head, const int32_t* head_map, int64_t N,
+                                   const int32_t* n_rows_dev, const int32_t* cand,
+                                   int64_t cand_stride, const int32_t* cand_len, const void* mask, int mask_dtype,
+                                   const int32_t* head_max_token, float scale, const float* q_scale,
+                                   const float* k_scale, const float* v_scale, void* stream) {
+  return sparse_attn_run(q, k, v, in_dtype, out, out_dtype, H, T, D, token_idx, row_head, head_map, N, n_rows_dev, cand,
+                         cand_stride, cand_len, mask, mask_dtype, head_max_token, scale, q_scale, k_scale, v_scale,
+                         nullptr, stream);
+}
+
+extern "C" int pfa_sparse_attn_fwd_ws(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, int in_dtype, pfa_tensor4 out,
+                                      int out_dtype, int H, int64_t T, int D, const int32_t* token_idx,
+                                      const int32_t* row_head, const int32_t* head_map, int64_t N,
+                                      const int32_t* n_rows_dev, const int32_t* cand, int64_t cand_stride,
+                                      const int32_t* cand_len, const void* mask, int mask_dtype,
+                                      const int32_t* head_max_token, float scale, const float* q_scale,
+                                      const float* k_scale, const float* v_scale, void* workspace, size_t ws_bytes,
+                                      void* stream) {
+  if (workspace != nullptr && ws_bytes < (size_t)((N > 0 ? N : 0) + 15) / 16) {
+    clear_error();
+    set_error("pfa_sparse_attn_fwd_ws: workspace of %zu bytes for %lld rows", ws_bytes, (long long)N);
+    return PFA_E_WORKSPACE;
+  }
+  return sparse_attn_run(q, k, v, in_dtype, out, out_dtype, H, T, D, token_idx, row_head, head_map, N, n_rows_dev, cand,
+                         cand_stride, cand_len, mask, mask_dtype, head_max_token, scale, q_scale, k_scale, v_scale,
+                         (uint8_t*)workspace, stream);
 }

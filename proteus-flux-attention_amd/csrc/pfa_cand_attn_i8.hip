@@ -1,0 +1,8 @@
+// The candidate attention kernel (pfa_cand_attn.h) for i8 inputs.
+#include "pfa_cand_attn.h"
+
+namespace pfa {
+int cand_attn_launch_i8(const AttnArgs& a, int out_dtype, int D, hipStream_t s) {
+  return cand::launch<PFA_I8>(a, out_dtype, D, s);
+}
+}  // namespace pfa

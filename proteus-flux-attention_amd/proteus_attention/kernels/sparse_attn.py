@@ -371,15 +371,16 @@ def _attn_launch(
 ) -> None:
     lib = _hip.lib()
     mask_tag = _hip.dtype_tag(mask.dtype) if mask is not None else 0
+    ws = _workspace((int(token_idx.numel()) + 15) // 16, device) if cand is not None and mask is None else None
     with _hip.TIMER.timed("sparse_attn_fwd"):
-        rc = lib.pfa_sparse_attn_fwd(
+        rc = lib.pfa_sparse_attn_fwd_ws(
         q4, k4, v4, _hip.dtype_tag(in_dtype), out4, _hip.dtype_tag(out_dtype), int(H), int(T), int(D),
         _hip.ptr(token_idx), _hip.ptr(row_head), _hip.ptr(head_map), int(token_idx.numel()), _hip.ptr(n_rows_dev),
         _hip.ptr(cand),
         int(cand.stride(0)) if cand is not None else 0, _hip.ptr(cand_len), _hip.ptr(mask), mask_tag,
         _hip.ptr(head_max), float(scale), _hip.ptr(scales[0]), _hip.ptr(scales[1]), _hip.ptr(scales[2]),
-        _hip.stream_ptr(device))
-    _hip.check(rc, "pfa_sparse_attn_fwd")
+        _hip.ptr(ws), ws.numel() if ws is not None else 0, _hip.stream_ptr(device))
+    _hip.check(rc, "pfa_sparse_attn_fwd_ws")
 
 
 def shortlist_partials(N: int, device: torch.device, D: int = 64) -> torch.Tensor:
