@@ -80,7 +80,8 @@ def _pack_mask_i32(mask_bool: torch.Tensor):
     lib = _hip.lib()
     device = mask_bool.device
     P, T = mask_bool.shape
-    m8 = mask_bool.to(torch.uint8).contiguous()
+    mask_bool = mask_bool.contiguous()
+    m8 = mask_bool.view(torch.uint8) if mask_bool.dtype == torch.bool else mask_bool.to(torch.uint8)
     ws = _workspace(_size_out(lib.pfa_pack_workspace_size, 1, P, T), device)
     row_offsets = torch.empty(P + 1, dtype=torch.int32, device=device)
     token_idx = torch.empty(P * T, dtype=torch.int32, device=device)

@@ -72,10 +72,11 @@ _SIDE_STREAMS: Dict[Tuple[int, str], torch.cuda.Stream] = {}
 #   bf16 shortlist, T = 1,024: 273 / 396; 16,384: 271 / 420; 40,960: 421 / 463;
 #     49,152: 482 / 425; 98,304: 711 / 663
 #   bf16 int8, 2 x 8,192: 370 / 476; 32,768: 428 / 504
-#   f32 shortlist, T = 4,096: 302 / 354; 6,000: 401 / 404; 10,007: 576 / 554
-#   f16 shortlist, T = 8,192: 336 / 408; 16,384: 516 / 510
+#   f32 shortlist, T = 4,096: 300 / 368; 6,000: 406 / 393; 8,192: 464 / 464;
+#     10,007: 597 / 568
+#   f16 shortlist, T = 8,192: 324 / 406; 16,384: 531 / 529; 24,576: 815 / 757
 # f32 and f16 layers attend gathered candidates and keep the device longer.
-_ONE_STREAM_ELEMS = {torch.bfloat16: 21 << 20, torch.float16: 4 << 20, torch.float32: 3 << 20}
+_ONE_STREAM_ELEMS = {torch.bfloat16: 21 << 20, torch.float16: 6 << 20, torch.float32: 5 << 19}
 
 
 def _side_stream(device: torch.device, role: str) -> torch.cuda.Stream:
