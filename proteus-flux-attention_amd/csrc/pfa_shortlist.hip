@@ -188,13 +188,70 @@ __device__ __forceinline__ uint64_t block_select(int n, int need, Get get, uint3
   return pval;
 }
 
-// Bitonic sort of cap = NT*V (V a power of two, 1..16) keys in LDS, largest
-// first, by a workgroup of NT threads.  Thread t holds the V keys
-// [V*t, V*t + V) in registers: strides below V are exchanged in registers,
-// strides below 64*V with the partner lane of the same wave (shuffles), and
-// the larger strides through LDS between barriers.  The caller has made the
-// keys visible to every thread (a barrier) before the call; they are in LDS,
-// sorted, and visible to every thread on return.
+// The value of lane (lane ^ LM): DPP within rows of sixteen lanes (xor 4 is
+// xor 7, the half-row mirror, then xor 3), through LDS across rows.  Every
+// lane of the wave is active.
+template <int LM>
+__device__ __forceinline__ uint32_t lane_xor32(uint32_t x) {
+  if constexpr (LM == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);
+  else if constexpr (LM == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);
+  else if constexpr (LM == 4) {
+    const int y = __builtin_amdgcn_update_dpp(0, (int)x, 0x141, 0xf, 0xf, true);
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, y, 0x1B, 0xf, 0xf, true);
+  } else if constexpr (LM == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, true);
+  else return (uint32_t)__shfl_xor((int)x, LM, 64);
+}
+template <int LM>
+__device__ __forceinline__ uint64_t lane_xor64(uint64_t x) {
+  return (uint64_t)lane_xor32<LM>((uint32_t)x) | ((uint64_t)lane_xor32<LM>((uint32_t)(x >> 32)) << 32);
+}
+
+// The strides JJ, JJ/2, .. 1 of the bitonic merge of KK keys; thread t of the
+// wave holds keys [V*t, V*t + V).  The last merge, of the wave's 64*V keys,
+// leaves them largest first in every wave.
+template <int V, int KK, int JJ>
+__device__ __forceinline__ void wave_merge(uint64_t (&r)[V], int tid) {
+  if constexpr (JJ >= V) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const uint64_t x = r[i], y = lane_xor64<JJ / V>(x);
+      const int e = V * tid + i;
+      const bool desc = KK == 64 * V || (e & KK) == 0, lower = (e & JJ) == 0;
+      const uint64_t hi = x > y ? x : y, lo = x > y ? y : x;
+      r[i] = (lower == desc) ? hi : lo;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      if ((i & JJ) == 0) {
+        const bool desc = KK == 64 * V || ((V * tid + i) & KK) == 0;
+        const uint64_t x = r[i], y = r[i | JJ];
+        const uint64_t hi = x > y ? x : y, lo = x > y ? y : x;
+        r[i] = desc ? hi : lo;
+        r[i | JJ] = desc ? lo : hi;
+      }
+    }
+  }
+  if constexpr (JJ > 1) wave_merge<V, KK, JJ / 2>(r, tid);
+}
+template <int V, int KK = 2>
+__device__ __forceinline__ void wave_sort_desc(uint64_t (&r)[V], int tid) {
+  wave_merge<V, KK, KK / 2>(r, tid);
+  if constexpr (KK < 64 * V) wave_sort_desc<V, 2 * KK>(r, tid);
+}
+
+// Sort of cap = NT*V (V a power of two) keys in LDS, largest first, by a
+// workgroup of NT threads.  Each wave sorts 64*V keys in registers (bitonic,
+// strides by DPP); the runs are then merged in pairs, log2(NT/64) rounds of
+// two barriers, each key finding its place by a binary search of the other
+// run (on equal keys the earlier run's comes first, so places are distinct).
+// Bound by the chain of dependent exchanges: a bitonic network across the
+// workgroup has 55 of them for 1,024 keys, 45 through LDS shuffles and 10
+// between barriers; here 21 in the wave (18 by DPP) and 34 probes.  At 8
+// superblocks of 1,024: prefix_sb_sort 13.6 -> 7.3 us, prefix_sb_prefix
+// 18.0 -> 11.8 us.
+// The caller has made the keys visible to every thread (a barrier) before the
+// call; they are in LDS, sorted, and visible to every thread on return.
 template <int NT, int V>
 __device__ __forceinline__ void block_sort_desc_v(uint64_t* k) {
   constexpr int cap = NT * V;
@@ -202,57 +259,33 @@ __device__ __forceinline__ void block_sort_desc_v(uint64_t* k) {
   uint64_t r[V];
 #pragma unroll
   for (int i = 0; i < V; ++i) r[i] = k[V * tid + i];
-  for (int kk = 2; kk <= cap; kk <<= 1) {
-    // strides of V and more: partner lanes (shuffles) or other waves (LDS)
-    for (int jj = kk >> 1; jj >= V; jj >>= 1) {
-      if (jj < 64 * V) {
-        const int lm = jj / V;  // partner lane distance (a power of two below 64)
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-          const uint64_t x = r[i];
-          const uint64_t y = __shfl_xor((unsigned long long)x, lm, 64);
-          const int e = V * tid + i;
-          const bool desc = (e & kk) == 0, lower = (e & jj) == 0;
-          const uint64_t hi = x > y ? x : y, lo = x > y ? y : x;
-          r[i] = (lower == desc) ? hi : lo;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < V; ++i) k[V * tid + i] = r[i];
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-          const int e = V * tid + i;
-          const uint64_t x = r[i], y = k[e ^ jj];
-          const bool desc = (e & kk) == 0, lower = (e & jj) == 0;
-          const uint64_t hi = x > y ? x : y, lo = x > y ? y : x;
-          r[i] = (lower == desc) ? hi : lo;
-        }
-        __syncthreads();
-      }
-    }
-    // strides below V: inside the thread's registers (static indices)
-#pragma unroll
-    for (int jj = V >> 1; jj >= 1; jj >>= 1) {
-      if (jj < kk) {
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-          if ((i & jj) == 0) {
-            const int pi = i | jj;
-            const int e = V * tid + i;
-            const bool desc = (e & kk) == 0;
-            const uint64_t x = r[i], y = r[pi];
-            const uint64_t hi = x > y ? x : y, lo = x > y ? y : x;
-            r[i] = desc ? hi : lo;
-            r[pi] = desc ? lo : hi;
-          }
-        }
-      }
-    }
-  }
+  wave_sort_desc<V>(r, tid);
 #pragma unroll
   for (int i = 0; i < V; ++i) k[V * tid + i] = r[i];
   __syncthreads();
+  for (int L = 64 * V; L < cap; L <<= 1) {
+    int at[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int e = NT * i + tid;
+      r[i] = k[e];
+      const bool second = (e & L) != 0;
+      const uint64_t* o = k + ((e & ~(L - 1)) ^ L);  // the other run
+      // keys of the other run that go before this one: those above it, and
+      // from the second run's view those equal to it as well
+      const uint64_t lim = r[i] - (second ? 1ull : 0ull);
+      const bool all = second && r[i] == 0ull;  // every key is >= 0
+      int pos = 0;
+      for (int h = L >> 1; h >= 1; h >>= 1)
+        if (o[pos + h - 1] > lim) pos += h;
+      if (o[pos] > lim) ++pos;
+      at[i] = (e & ~(2 * L - 1)) + (e & (L - 1)) + (all ? L : pos);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < V; ++i) k[at[i]] = r[i];
+    __syncthreads();
+  }
 }
 
 // Element p of top-K(a U c) for best-first (descending) key lists a (na)
