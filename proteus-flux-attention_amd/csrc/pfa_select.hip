@@ -699,8 +699,8 @@ extern "C" int pfa_pack_mask(const uint8_t* mask, int P, int64_t T, int32_t* row
   dim3 grid(nblk, (unsigned)P);
   pack_count_mask<<<grid, kPackThreads, 0, s>>>(mask, T, nblk, w.blockcounts);
   PFA_CHECK_LAUNCH("pfa_pack_mask/count");
-  // two launches instead of three: 8 x 4,096 rows, the f16 causal operator
-  // 115 -> 105 us a call with the mask read in place
+  // two launches instead of three: the f16 causal operator at 16 heads x
+  // 4,096 tokens 115 -> 105 us a call, with the mask read in place
   if ((int64_t)P * nblk <= kFusedScanMax) {
     pack_fill_scan_kernel<<<grid, kPackThreads, (size_t)P * sizeof(int), s>>>(
         mask, P, T, nblk, w.blockcounts, 0, nullptr, row_offsets_out, summary_out, token_idx_out, row_head_out, nullptr);

@@ -18,7 +18,8 @@ packing (1704-1756)                    ``pfa_pack_rows``
 shortlist candidates (1269-1284)       ``pfa_proto_prefix_topk`` + ``pfa_shortlist_build``
 sparse attention + scatter (1287-1302,
 1802-1807, 1841-1842)                  ``pfa_sparse_attn_fwd`` writing (B,T,H,D)
-prototype EMA (692-718)                ``pfa_proto_accumulate`` + reduce
+prototype EMA (692-718)                sums in the router or ``pfa_proto_accumulate``,
+                                       then ``pfa_router_tail``
 =====================================  ======================================
 
 The attention kernel reads q/k/v straight out of the (B, T, 3, H, D) QKV
