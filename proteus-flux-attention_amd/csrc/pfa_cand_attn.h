@@ -14,10 +14,10 @@
 //
 // The row kernel fetches K and V once per (row, candidate) and multiplies on
 // the vector unit; here they are fetched once per (sixteen rows, key).
-// 16,400 rows of 8 heads x 64 dims, T = 8,192, 393 candidates a row: bf16 134
-// -> 55 us, f32 143 -> 86 us.  Bound by latency: marking and listing a
+// 16,400 rows of 8 heads x 64 dims, T = 8,192, 393 candidates a row: bf16 132
+// -> 49 us, f32 139 -> 88 us.  Bound by latency: marking and listing a
 // workgroup's keys takes about half of it, two workgroups fit a CU (72 KB of
-// LDS, 240 VGPRs), and a tile's keys are gathered one tile ahead.
+// LDS, up to 256 VGPRs), and a tile's keys are gathered one tile ahead.
 #pragma once
 
 #include "pfa_tile_attn.h"
@@ -25,11 +25,19 @@
 namespace pfa {
 namespace cand {
 
+using tile::exp2_p;
 using tile::f32_swz;
-using tile::kPShift;
+using tile::i8_bf16;
+using tile::kFused;
+using tile::kParts;
+using tile::kPScale;
 using tile::mfma16;
+using tile::negate_q;
+using tile::normalise;
+using tile::products_f32;
 using tile::split_p;
 using tile::store_n;
+using tile::tree_sum;
 
 constexpr int kRange = 8192;  // keys marked at a time
 constexpr int kCap = 4096;    // listed keys between two flushes
@@ -113,12 +121,8 @@ cand_attn_kernel(AttnArgs a, int odt) {
         qf[dc] = bf16x8_t{};
         if (D >= 32 || g < 2) {
           if constexpr (IDT == PFA_I8) {
-            float x[8];
-            load8<PFA_I8>(qp + 32 * dc + 8 * g, x);
-            _Float16 h[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) h[i] = (_Float16)x[i];
-            __builtin_memcpy(&qf[dc], h, 16);
+            const uint2 w = *reinterpret_cast<const uint2*>(qp + 32 * dc + 8 * g);
+            qf[dc] = i8_bf16(w.x, w.y);
           } else {
             qf[dc] = *reinterpret_cast<const bf16x8_t*>(qp + 32 * dc + 8 * g);
           }
@@ -127,6 +131,10 @@ cand_attn_kernel(AttnArgs a, int odt) {
     }
     float sl2 = a.scale * kLog2e;
     if constexpr (IDT == PFA_I8) sl2 *= a.q_scale[bh] * a.k_scale[bh];
+    if (sl2 < 0.f) {  // (as in the tile kernel)
+      sl2 = -sl2;
+      negate_q<C::kF32>(qx, qf);
+    }
     float m = -INFINITY, l = 0.f;
     f32x4_t acc[NDB];
 #pragma unroll
@@ -176,39 +184,15 @@ cand_attn_kernel(AttnArgs a, int odt) {
         }
       }
     };
-    auto to_f16 = [](uint32_t x, uint32_t y) {
-      const uint32_t w[2] = {x, y};
-      _Float16 h[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) h[i] = (_Float16)(float)(int8_t)(w[i >> 2] >> (8 * (i & 3)));
-      bf16x8_t o;
-      __builtin_memcpy(&o, h, 16);
-      return o;
-    };
     auto compute = [&](int tile, int buf, const Regs& x) {
       f32x4_t c[NKB];
       if constexpr (C::kF32) {
-        constexpr int NC = D / 16 < 4 ? D / 16 : 4;  // chains, as in the tile kernel
-        f32x4_t cc[NC][NKB];
-#pragma unroll
-        for (int n = 0; n < NC; ++n)
-#pragma unroll
-          for (int b = 0; b < NKB; ++b) cc[n][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < D / 16; ++j)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int b = 0; b < NKB; ++b) {
-              f32x4_t kv;
-              __builtin_memcpy(&kv, &x.k[j][b], 16);
-              cc[j % NC][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], qx[j][i], cc[j % NC][b], 0, 0, 0);
-            }
 #pragma unroll
         for (int b = 0; b < NKB; ++b) {
-          if constexpr (NC == 4) c[b] = (cc[0][b] + cc[1][b]) + (cc[2][b] + cc[3][b]);
-          else if constexpr (NC == 2) c[b] = cc[0][b] + cc[1][b];
-          else c[b] = cc[0][b];
+          f32x4_t ka[D / 16];
+#pragma unroll
+          for (int j = 0; j < D / 16; ++j) __builtin_memcpy(&ka[j], &x.k[j][b], 16);
+          c[b] = products_f32<D / 16>([&](int n) { return ka[n >> 2][n & 3]; }, [&](int n) { return qx[n >> 2][n & 3]; });
         }
       } else {
 #pragma unroll
@@ -216,7 +200,7 @@ cand_attn_kernel(AttnArgs a, int odt) {
 #pragma unroll
           for (int b = 0; b < NKB; ++b) {
             bf16x8_t ka;
-            if constexpr (IDT == PFA_I8) ka = to_f16(x.k[dc][b].x, x.k[dc][b].y);
+            if constexpr (IDT == PFA_I8) ka = i8_bf16(x.k[dc][b].x, x.k[dc][b].y);
             else __builtin_memcpy(&ka, &x.k[dc][b], 16);
             c[b] = mfma16<IDT>(ka, qf[dc], dc == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : c[b]);
           }
@@ -225,13 +209,13 @@ cand_attn_kernel(AttnArgs a, int odt) {
 #pragma unroll
         for (int j = 0; j < kVr; ++j) {
           const int n = lane + 64 * j, row = n / (D / 8), ch = n % (D / 8);
-          const bf16x8_t h = to_f16(x.v[j].x, x.v[j].y);
+          const bf16x8_t h = i8_bf16(x.v[j].x, x.v[j].y);
           __builtin_memcpy(__builtin_assume_aligned(&vring[wid][buf][(ch >> 3) * TK * 128 + row * 128 +
                                                                       16 * ((ch & 7) ^ tile_swz(row))], 16), &h, 16);
         }
         wave_sync();
       }
-      // scores in log2 units; -inf where the row does not list the key
+      // scores (unscaled where kFused); -inf where the row does not list the key
       float s[NKB][4], tmax = -INFINITY;
 #pragma unroll
       for (int b = 0; b < NKB; ++b) {
@@ -239,14 +223,15 @@ cand_attn_kernel(AttnArgs a, int odt) {
         const uint32_t mk[4] = {mw.x, mw.x >> 16, mw.y, mw.y >> 16};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          s[b][i] = (mk[i] >> r16) & 1u ? c[b][i] * sl2 : -INFINITY;
+          s[b][i] = (mk[i] >> r16) & 1u ? (kFused<IDT> ? c[b][i] : c[b][i] * sl2) : -INFINITY;
           tmax = fmaxf(tmax, s[b][i]);
         }
       }
       tmax = max_over_rows4(tmax);
+      if constexpr (kFused<IDT>) tmax *= sl2;  // sl2 > 0, -inf stays
       if (__ballot(tmax > m) != 0) {
         const float mn = fmaxf(m, tmax);
-        const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+        const float alpha = mn == -INFINITY ? 1.f : exp2_p<IDT>(m - mn);
         l *= alpha;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
@@ -254,43 +239,38 @@ cand_attn_kernel(AttnArgs a, int odt) {
           for (int i = 0; i < 4; ++i) acc[db][i] *= alpha;
         m = mn;
       }
-      const float moff = (m == -INFINITY ? 0.f : m) - kPShift<IDT>;
-      float ps = 0.f;
+      const float moff = m == -INFINITY ? 0.f : m;
+      float ps[NKB];
 #pragma unroll
-      for (int b = 0; b < NKB; ++b)
+      for (int b = 0; b < NKB; ++b) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          s[b][i] = __builtin_amdgcn_exp2f(s[b][i] - moff);
-          ps += s[b][i];
+          const float x = kFused<IDT> ? __builtin_fmaf(s[b][i], sl2, -moff) : s[b][i] - moff;
+          s[b][i] = exp2_p<IDT>(x) * kPScale<IDT>;
         }
-      l += ps;
+        ps[b] = (s[b][0] + s[b][1]) + (s[b][2] + s[b][3]);
+      }
+      l += tree_sum(ps);
       if constexpr (C::kF32) {
         const float* vt = (const float*)&vring[wid][buf][0];
-        f32x4_t ta[NDB];
+        float va[4 * NKB][NDB];
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) ta[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int n = 0; n < 4 * NKB; ++n) {
+          const int row = 16 * (n >> 2) + 4 * g + (n & 3);
+          const float* vr = vt + row * D;
+          if constexpr (NDB >= 4) {
 #pragma unroll
-        for (int b = 0; b < NKB; ++b)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int row = 16 * b + 4 * g + i;
-            const float* vr = vt + row * D;
-            float va[NDB];
-            if constexpr (NDB >= 4) {
-#pragma unroll
-              for (int h = 0; h < NDB / 4; ++h)
-                __builtin_memcpy(va + 4 * h, __builtin_assume_aligned(vr + 4 * ((16 * h + r16) ^ f32_swz<D>(row)), 16), 16);
-            } else {
-              const int d0 = NDB * r16;
-              __builtin_memcpy(va, __builtin_assume_aligned(vr + 4 * ((d0 >> 2) ^ f32_swz<D>(row)) + (d0 & 3), 4 * NDB),
-                               4 * NDB);
-            }
-#pragma unroll
-            for (int db = 0; db < NDB; ++db)
-              ta[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[db], s[b][i], ta[db], 0, 0, 0);
+            for (int h = 0; h < NDB / 4; ++h)
+              __builtin_memcpy(va[n] + 4 * h, __builtin_assume_aligned(vr + 4 * ((16 * h + r16) ^ f32_swz<D>(row)), 16), 16);
+          } else {
+            const int d0 = NDB * r16;
+            __builtin_memcpy(va[n], __builtin_assume_aligned(vr + 4 * ((d0 >> 2) ^ f32_swz<D>(row)) + (d0 & 3), 4 * NDB),
+                             4 * NDB);
           }
+        }
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) acc[db] += ta[db];
+        for (int db = 0; db < NDB; ++db)
+          acc[db] += products_f32<NKB>([&](int n) { return va[n][db]; }, [&](int n) { return s[n >> 2][n & 3]; });
       } else {
         const uint16_t* vt = (const uint16_t*)&vring[wid][buf][0];
         float p[8];
@@ -299,8 +279,8 @@ cand_attn_kernel(AttnArgs a, int odt) {
           p[i] = s[0][i];
           p[4 + i] = s[NKB - 1][i];
         }
-        bf16x8_t hi, lo;
-        split_p<IDT>(p, hi, lo);
+        bf16x8_t part[kParts];
+        split_p<IDT>(p, part);
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
           const uint16_t* vr = vt + (db >> 2) * TK * 64 + L.vo[db & 3];
@@ -308,8 +288,8 @@ cand_attn_kernel(AttnArgs a, int odt) {
           bf16x8_t va;
           __builtin_memcpy(&va, &v0, 8);
           __builtin_memcpy(reinterpret_cast<char*>(&va) + 8, &v1, 8);
-          acc[db] = mfma16<IDT>(va, hi, acc[db]);
-          acc[db] = mfma16<IDT>(va, lo, acc[db]);
+#pragma unroll
+          for (int n = kParts - 1; n >= 0; --n) acc[db] = mfma16<IDT>(va, part[n], acc[db]);
         }
       }
     };
@@ -504,8 +484,8 @@ cand_attn_kernel(AttnArgs a, int odt) {
       for (int k = 0; k < 3; ++k) {
         const float* o = area + k * W * 64 + lane;
         const float mo = o[0], mn = fmaxf(m, mo);
-        const float fa = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
-        const float fb = mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - mn);
+        const float fa = m == -INFINITY ? 0.f : exp2_p<IDT>(m - mn);
+        const float fb = mo == -INFINITY ? 0.f : exp2_p<IDT>(mo - mn);
         l = l * fa + o[64] * fb;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
@@ -513,14 +493,14 @@ cand_attn_kernel(AttnArgs a, int odt) {
           for (int i = 0; i < 4; ++i) acc[db][i] = acc[db][i] * fa + o[64 * (2 + 4 * db + i)] * fb;
         m = mn;
       }
-      float inv = 1.f / l;
-      if constexpr (IDT == PFA_I8) inv *= a.v_scale[bh];
       bool bad = false;
+      const float inv = 1.f / l;
+      const float vs = IDT == PFA_I8 ? a.v_scale[bh] : 1.f;
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          acc[db][i] *= inv;
+          acc[db][i] = normalise<IDT>(acc[db][i], l, inv, vs);
           bad |= !(fabsf(acc[db][i]) <= 3.402823466e38f);
           if (l == 0.f) acc[db][i] = __builtin_nanf("");  // every score -inf, or no candidate
         }

@@ -8,20 +8,24 @@
 // one query row (lane mod 16) and, of every 16-key block, the keys
 // 4 (lane/16) ..+3.  The row kernel (pfa_attn.hip) reads every key from cache
 // again for each row and multiplies on the vector unit.  At 16 heads x 4,096
-// tokens x 64 dims, half the rows active, f16 causal: 922 -> 76 us (225
-// TFLOP/s; bound by the softmax's vector work, two P.V products beside it).
-// 16 heads x 1,500 tokens, f32 masked: 409 -> 95 us (49 TFLOP/s of the 154
+// tokens x 64 dims, half the rows active, f16 causal: 815 -> 81 us (213
+// TFLOP/s; bound by the softmax's vector work, three P.V products beside it).
+// 16 heads x 1,500 tokens, f32 masked: 377 -> 98 us (47 TFLOP/s of the 154
 // that a large f32 product reaches; 188 blocks of rows do not fill the chip).
 //
-// Precision is the row kernel's: scores and softmax in f32, and P.V products
-// with P at f32 precision.
-//   f32  : v_mfma_f32_16x16x4_f32 for both products (f32 throughout).
-//   16-bit inputs: QK^T products are exact in f32; P is split into two parts of
-//     the input type (hi = round(P), lo = round(P - hi)), two products per
-//     tile.  f16 parts of 4096 P carry 22 bits of it; bf16 parts carry 16
-//     bits, well below the rounding of the bf16 result.
-//   int8 : values are exact in f16 (converted on the way into LDS), P as for
-//     f16; the per-head scales ride on the score scale and the output.
+// Scores, softmax and sums are f32, and P keeps all 24 bits of its f32 value:
+//   f32  : v_mfma_f32_16x16x4_f32 (four fma in turn) for both products, in
+//     short sums (products_f32).
+//   16-bit inputs: QK^T products are exact in f32; P is split into three parts
+//     of the input type (split_p), three products per tile.
+//   int8 : values are exact in bf16 (converted on the way into LDS), P as for
+//     bf16; the per-head scales ride on the score scale and the output.
+// Two things are below the row kernel: f16 inputs hold P to 2^-39 absolutely
+// where it is under 2^-16, and with 16-bit and int8 inputs a P under 2^-126
+// counts as zero.  Distance from the 64-bit result over lengths of 16 to 400
+// (24 draws each), of the row kernel's: f32 0.85-0.99, int8 0.57-0.76; with P
+// in two 16-bit parts and longer sums int8 was at 1.4-1.6 and f32 at 1.1-1.4,
+// for 4-19% less time.
 //
 // KS = 4/RG key splits: with few rows the four waves of a workgroup share
 // fewer row groups and take every KS-th tile each; their partial states meet
@@ -71,10 +75,11 @@ __device__ __forceinline__ int f32_swz(int r) {
   else return (r >> 2) & 3;
 }
 
-// bf16 products for bf16 inputs, f16 products otherwise (f16 and int8).
+// f16 products for f16 inputs, bf16 products for bf16 and int8 (whose values
+// are exact in bf16).
 template <int IDT>
 __device__ __forceinline__ f32x4_t mfma16(bf16x8_t a, bf16x8_t b, f32x4_t c) {
-  if constexpr (IDT == PFA_BF16) {
+  if constexpr (IDT != PFA_F16) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   } else {
     f16x8_t x, y;
@@ -84,35 +89,129 @@ __device__ __forceinline__ f32x4_t mfma16(bf16x8_t a, bf16x8_t b, f32x4_t c) {
   }
 }
 
-// P (8 values) as hi + lo parts of the product type.  The f16 form comes with
-// 4096 P (kPShift rides in the exponent, and the row sum with it): hi is cut
-// off, lo = round(P - hi) is exact to 2^-22 P and to 2^-36 absolutely.
+// P (8 values) as kParts parts of the product type, each cut off from what
+// the parts before it leave: all 24 bits of P.  bf16 parts carry 8 bits each
+// at any size; f16 parts 11, of kPScale P (and the row sum with it), so that P
+// has its 24 bits down to 2^-16 and 2^-39 absolutely below.  The scale is
+// multiplied on: in the exponent it would cost the exponent's own last bits.
+constexpr int kParts = 3;
 template <int IDT>
-constexpr float kPShift = IDT == PFA_F16 || IDT == PFA_I8 ? 12.f : 0.f;
+constexpr float kPScale = IDT == PFA_F16 ? 32768.f : 1.f;
 template <int IDT>
-__device__ __forceinline__ void split_p(const float (&p)[8], bf16x8_t& hi, bf16x8_t& lo) {
-  if constexpr (IDT == PFA_BF16) {
-    __bf16 h[8], l[8];
+__device__ __forceinline__ void split_p(const float (&p)[8], bf16x8_t (&part)[kParts]) {
+  float r[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      h[i] = (__bf16)p[i];
-      l[i] = (__bf16)(p[i] - (float)h[i]);
-    }
-    __builtin_memcpy(&hi, h, 16);
-    __builtin_memcpy(&lo, l, 16);
-  } else {
-    _Float16 l[8];
-    f16x2_t h[4];
+  for (int i = 0; i < 8; ++i) r[i] = p[i];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const auto w = __builtin_amdgcn_cvt_pkrtz(p[2 * i], p[2 * i + 1]);
-      __builtin_memcpy(&h[i], &w, 4);
-      l[2 * i] = (_Float16)(p[2 * i] - (float)h[i][0]);
-      l[2 * i + 1] = (_Float16)(p[2 * i + 1] - (float)h[i][1]);
+  for (int n = 0; n < kParts; ++n) {
+    if constexpr (IDT == PFA_F16) {
+      f16x2_t h[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const auto w = __builtin_amdgcn_cvt_pkrtz(r[2 * i], r[2 * i + 1]);
+        __builtin_memcpy(&h[i], &w, 4);
+        r[2 * i] -= (float)h[i][0];
+        r[2 * i + 1] -= (float)h[i][1];
+      }
+      __builtin_memcpy(&part[n], h, 16);
+    } else {
+      uint32_t h[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t a = __float_as_uint(r[2 * i]), b = __float_as_uint(r[2 * i + 1]);
+        h[i] = __builtin_amdgcn_perm(b, a, 0x07060302u);  // their upper halves
+        r[2 * i] -= __uint_as_float(a & 0xffff0000u);
+        r[2 * i + 1] -= __uint_as_float(b & 0xffff0000u);
+      }
+      __builtin_memcpy(&part[n], h, 16);
     }
-    __builtin_memcpy(&hi, h, 16);
-    __builtin_memcpy(&lo, l, 16);
   }
+}
+
+// 2^x of a probability or a factor of one.  f32 results keep the row kernel's
+// denormals.
+template <int IDT>
+__device__ __forceinline__ float exp2_p(float x) {
+  if constexpr (IDT == PFA_F32) return exp2f(x);
+  else return __builtin_amdgcn_exp2f(x);
+}
+
+// Whether a score is scaled in the step that takes it off its maximum.  The
+// maximum is a rounded product and the score then is not: at large scores it
+// can come out above it, P above 1, where f16 parts end (at 2^17 of 2^15 P).
+template <int IDT>
+constexpr bool kFused = IDT != PFA_F16;
+
+// int8 values as bf16
+__device__ __forceinline__ bf16x8_t i8_bf16(uint32_t x, uint32_t y) {
+  const uint32_t w[2] = {x, y};
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t v = w[i >> 1] >> (16 * (i & 1));
+    o[i] = __builtin_amdgcn_perm(__float_as_uint((float)(int8_t)(v >> 8)), __float_as_uint((float)(int8_t)v), 0x07060302u);
+  }
+  bf16x8_t b;
+  __builtin_memcpy(&b, o, 16);
+  return b;
+}
+
+template <bool FIRST, typename V>
+__device__ __forceinline__ V& pick(V& a, V& b) {
+  if constexpr (FIRST) return a;
+  else return b;
+}
+
+// A result from its sum: divided where it may be stored as f32, by the
+// reciprocal where 16 bits of it are.
+template <int IDT>
+__device__ __forceinline__ float normalise(float x, float l, float inv, float vs) {
+  if constexpr (IDT == PFA_F32) return x / l;
+  else if constexpr (IDT == PFA_I8) return x / l * vs;
+  else return x * inv;
+}
+
+// The query of a row, negated.
+template <bool F32, int NX, int NF>
+__device__ __forceinline__ void negate_q(f32x4_t (&qx)[NX], bf16x8_t (&qf)[NF]) {
+  if constexpr (F32) {
+#pragma unroll
+    for (int j = 0; j < NX; ++j) qx[j] = -qx[j];
+  } else {
+#pragma unroll
+    for (int dc = 0; dc < NF; ++dc) {
+      uint32_t w[4];
+      __builtin_memcpy(w, &qf[dc], 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] ^= 0x80008000u;
+      __builtin_memcpy(&qf[dc], w, 16);
+    }
+  }
+}
+
+// Sum of N (a power of two) values in a tree.
+template <int N, typename V>
+__device__ __forceinline__ V tree_sum(V (&x)[N]) {
+#pragma unroll
+  for (int w = 1; w < N; w *= 2)
+#pragma unroll
+    for (int i = 0; i + w < N; i += 2 * w) x[i] = x[i] + x[i + w];
+  return x[0];
+}
+
+// The f32 product over 4 N k-steps of four terms, a(n) b(n): sums of eight
+// terms, then a tree, so that no sum is longer than the row kernel's lanes
+// keep it.  (Sums of sixteen leave results of 32-dim heads 9% further from the
+// 64-bit ones than the row kernel's, and take 3% less time.)
+template <int N, typename A, typename B>
+__device__ __forceinline__ f32x4_t products_f32(A a, B b) {
+  f32x4_t part[2 * N];
+#pragma unroll
+  for (int n = 0; n < 2 * N; ++n) {
+    part[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a(2 * n), b(2 * n), f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    part[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a(2 * n + 1), b(2 * n + 1), part[n], 0, 0, 0);
+  }
+  return tree_sum(part);
 }
 
 // Store n consecutive output values (aligned to n elements).
@@ -200,7 +299,7 @@ tile_attn_kernel(AttnArgs a, int odt) {
 
     // ---- tiles into LDS: step st brings the tiles st*KS .. st*KS+KS-1 ----
     // f32 and 16-bit tiles go by LDS DMA (1 KB per wave and transfer); int8
-    // tiles through registers, converted to f16 on the way.
+    // tiles through registers, converted to bf16 on the way.
     // Thread tid moves the 16-byte slots tid + 256 j of each K or V tile; the
     // rows of j > 0 lie a multiple of 16 further (8 for f32 rows of 128), so
     // the chunk that belongs in the slot is the same for every j (but for the
@@ -253,13 +352,10 @@ tile_attn_kernel(AttnArgs a, int odt) {
         const int n = tid + 256 * j;
         const int c = n % CW, row = (n / CW) % TK, sub = (n / (CW * TK)) % KS;
         const int isv = n / (CW * TK * KS);
-        const uint32_t w[2] = {regs[j].x, regs[j].y};
-        _Float16 h[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) h[i] = (_Float16)(float)(int8_t)(w[i >> 2] >> (8 * (i & 3)));
+        const bf16x8_t h = i8_bf16(regs[j].x, regs[j].y);
         uint8_t* dst = stage + sub * C::kTileBytes + isv * C::kHalfBytes + (c >> 3) * TK * 128 + row * 128 +
                        16 * ((c & 7) ^ tile_swz(row));
-        __builtin_memcpy(__builtin_assume_aligned(dst, 16), h, 16);
+        __builtin_memcpy(__builtin_assume_aligned(dst, 16), &h, 16);
       }
     };
     if constexpr (IDT == PFA_I8) fetch8(0);
@@ -280,12 +376,8 @@ tile_attn_kernel(AttnArgs a, int odt) {
         qf[dc] = bf16x8_t{};
         if (D >= 32 || g < 2) {
           if constexpr (IDT == PFA_I8) {
-            float x[8];
-            load8<PFA_I8>(qp + 32 * dc + 8 * g, x);
-            _Float16 h[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) h[i] = (_Float16)x[i];
-            __builtin_memcpy(&qf[dc], h, 16);
+            const uint2 w = *reinterpret_cast<const uint2*>(qp + 32 * dc + 8 * g);
+            qf[dc] = i8_bf16(w.x, w.y);
           } else {
             qf[dc] = *reinterpret_cast<const bf16x8_t*>(qp + 32 * dc + 8 * g);
           }
@@ -295,22 +387,11 @@ tile_attn_kernel(AttnArgs a, int odt) {
     }
     float sl2 = a.scale * kLog2e;
     if constexpr (IDT == PFA_I8) sl2 *= a.q_scale[bh] * a.k_scale[bh];
-    if (!MASKED && sl2 < 0.f) {
-      // the maximum is taken over unscaled scores: negate q instead
+    if (sl2 < 0.f) {
+      // the maximum may be taken over unscaled scores (kFused): negate q
+      // instead
       sl2 = -sl2;
-      if constexpr (C::kF32) {
-#pragma unroll
-        for (int j = 0; j < D / 16; ++j) qx[j] = -qx[j];
-      } else {
-#pragma unroll
-        for (int dc = 0; dc < C::NDC; ++dc) {
-          uint32_t w[4];
-          __builtin_memcpy(w, &qf[dc], 16);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) w[i] ^= 0x80008000u;
-          __builtin_memcpy(&qf[dc], w, 16);
-        }
-      }
+      negate_q<C::kF32>(qx, qf);
     }
 
     float m = -INFINITY, l = 0.f;
@@ -373,34 +454,14 @@ tile_attn_kernel(AttnArgs a, int odt) {
         f32x4_t c[NKB];
         if constexpr (C::kF32) {
           const float* kt = (const float*)tb;
-          // up to four chains per key block (every NC-th 16-dim step): short
-          // sums, as the row kernel's lanes keep them, and independent
-          // products to issue
-          constexpr int NC = D / 16 < 4 ? D / 16 : 4;
-          f32x4_t cc[NC][NKB];
-#pragma unroll
-          for (int n = 0; n < NC; ++n)
-#pragma unroll
-            for (int b = 0; b < NKB; ++b) cc[n][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int j = 0; j < D / 16; ++j) {
-            f32x4_t ka[NKB];
-#pragma unroll
-            for (int b = 0; b < NKB; ++b) {
-              const int row = 16 * b + r16;
-              ka[b] = *reinterpret_cast<const f32x4_t*>(kt + row * D + 4 * ((4 * j + g) ^ f32_swz<D>(row)));
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-              for (int b = 0; b < NKB; ++b)
-                cc[j % NC][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[b][i], qx[j][i], cc[j % NC][b], 0, 0, 0);
-          }
 #pragma unroll
           for (int b = 0; b < NKB; ++b) {
-            if constexpr (NC == 4) c[b] = (cc[0][b] + cc[1][b]) + (cc[2][b] + cc[3][b]);
-            else if constexpr (NC == 2) c[b] = cc[0][b] + cc[1][b];
-            else c[b] = cc[0][b];
+            const int row = 16 * b + r16;
+            f32x4_t ka[D / 16];
+#pragma unroll
+            for (int j = 0; j < D / 16; ++j)
+              ka[j] = *reinterpret_cast<const f32x4_t*>(kt + row * D + 4 * ((4 * j + g) ^ f32_swz<D>(row)));
+            c[b] = products_f32<D / 16>([&](int n) { return ka[n >> 2][n & 3]; }, [&](int n) { return qx[n >> 2][n & 3]; });
           }
         } else {
           const uint16_t* kt = (const uint16_t*)tb;
@@ -426,17 +487,18 @@ tile_attn_kernel(AttnArgs a, int odt) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             float x = c[b][i];
-            if constexpr (MASKED) x = __builtin_fmaf(mc[b][i], kLog2e, x * sl2);
+            if constexpr (MASKED) x = __builtin_fmaf(x, sl2, kLog2e * mc[b][i]);
+            else if constexpr (!kFused<IDT>) x *= sl2;
             if (cut && 16 * b + i > last) x = -INFINITY;
             s[b][i] = x;
             tmax = fmaxf(tmax, x);
           }
         }
         tmax = max_over_rows4(tmax);
-        if constexpr (!MASKED) tmax *= sl2;  // sl2 > 0, -inf stays
+        if constexpr (!MASKED && kFused<IDT>) tmax *= sl2;  // sl2 > 0, -inf stays
         if (__ballot(tmax > m) != 0) {  // some row's maximum rises
           const float mn = fmaxf(m, tmax);
-          const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+          const float alpha = mn == -INFINITY ? 1.f : exp2_p<IDT>(m - mn);
           l *= alpha;
 #pragma unroll
           for (int db = 0; db < NDB; ++db)
@@ -444,49 +506,52 @@ tile_attn_kernel(AttnArgs a, int odt) {
             for (int i = 0; i < 4; ++i) acc[db][i] *= alpha;
           m = mn;
         }
-        const float moff = (m == -INFINITY ? 0.f : m) - kPShift<IDT>;  // m = -inf: only -inf scores so far
-        float ps = 0.f;
+        const float moff = m == -INFINITY ? 0.f : m;  // m = -inf: only -inf scores so far
+        float ps[NKB];
 #pragma unroll
-        for (int b = 0; b < NKB; ++b)
+        for (int b = 0; b < NKB; ++b) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            s[b][i] = __builtin_amdgcn_exp2f(MASKED ? s[b][i] - moff : __builtin_fmaf(s[b][i], sl2, -moff));
-            ps += s[b][i];
+            const float x = MASKED || !kFused<IDT> ? s[b][i] - moff : __builtin_fmaf(s[b][i], sl2, -moff);
+            s[b][i] = exp2_p<IDT>(x) * kPScale<IDT>;
           }
-        l += ps;
+          ps[b] = (s[b][0] + s[b][1]) + (s[b][2] + s[b][3]);
+        }
+        l += tree_sum(ps);
         if constexpr (C::kF32) {
           // V^T rows are the dims NDB * m + db (db < 4; the second 64 dims
           // for db >= 4): one read per key serves every db.  A tile's products
           // are summed by themselves and then added, so that the sums stay
-          // short (as the row kernel's eight key groups keep them)
-          f32x4_t ta[NDB];
-#pragma unroll
-          for (int db = 0; db < NDB; ++db) ta[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          // short
           const float* vt = (const float*)(tb + C::kHalfBytes);
+          float va[4 * NKB][NDB];
 #pragma unroll
-          for (int b = 0; b < NKB; ++b)
+          for (int n = 0; n < 4 * NKB; ++n) {
+            const int row = 16 * (n >> 2) + 4 * g + (n & 3);
+            const float* vr = vt + row * D;
+            if constexpr (NDB >= 4) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int row = 16 * b + 4 * g + i;
-              const float* vr = vt + row * D;
-              float va[NDB];
-              if constexpr (NDB >= 4) {
-#pragma unroll
-                for (int h = 0; h < NDB / 4; ++h)
-                  __builtin_memcpy(va + 4 * h, __builtin_assume_aligned(vr + 4 * ((16 * h + r16) ^ f32_swz<D>(row)), 16), 16);
-              } else {
-                const int d0 = NDB * r16;
-                __builtin_memcpy(va, __builtin_assume_aligned(vr + 4 * ((d0 >> 2) ^ f32_swz<D>(row)) + (d0 & 3), 4 * NDB),
-                                 4 * NDB);
-              }
-#pragma unroll
-              for (int db = 0; db < NDB; ++db)
-                ta[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[db], s[b][i], ta[db], 0, 0, 0);
+              for (int h = 0; h < NDB / 4; ++h)
+                __builtin_memcpy(va[n] + 4 * h, __builtin_assume_aligned(vr + 4 * ((16 * h + r16) ^ f32_swz<D>(row)), 16),
+                                 16);
+            } else {
+              const int d0 = NDB * r16;
+              __builtin_memcpy(va[n], __builtin_assume_aligned(vr + 4 * ((d0 >> 2) ^ f32_swz<D>(row)) + (d0 & 3), 4 * NDB),
+                               4 * NDB);
             }
+          }
 #pragma unroll
-          for (int db = 0; db < NDB; ++db) acc[db] += ta[db];
+          for (int db = 0; db < NDB; ++db)
+            acc[db] += products_f32<NKB>([&](int n) { return va[n][db]; }, [&](int n) { return s[n >> 2][n & 3]; });
         } else {
           const uint16_t* vt = (const uint16_t*)(tb + C::kHalfBytes);
+          // (int8 results are f32: the tile by itself, as above)
+          f32x4_t ta[NDB];
+          auto& to = pick<IDT == PFA_I8>(ta, acc);
+          if constexpr (IDT == PFA_I8) {
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) ta[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
 #pragma unroll
           for (int kc = 0; kc < NKB / 2; ++kc) {
             float p[8];
@@ -495,8 +560,8 @@ tile_attn_kernel(AttnArgs a, int odt) {
               p[i] = s[2 * kc][i];
               p[4 + i] = s[2 * kc + 1][i];
             }
-            bf16x8_t hi, lo;
-            split_p<IDT>(p, hi, lo);
+            bf16x8_t part[kParts];
+            split_p<IDT>(p, part);
 #pragma unroll
             for (int db = 0; db < NDB; ++db) {
               const uint16_t* vr = vt + (db >> 2) * TK * 64 + 64 * 32 * kc + L.vo[db & 3];
@@ -504,9 +569,13 @@ tile_attn_kernel(AttnArgs a, int odt) {
               bf16x8_t va;
               __builtin_memcpy(&va, &v0, 8);
               __builtin_memcpy(reinterpret_cast<char*>(&va) + 8, &v1, 8);
-              acc[db] = mfma16<IDT>(va, hi, acc[db]);
-              acc[db] = mfma16<IDT>(va, lo, acc[db]);
+#pragma unroll
+              for (int n = kParts - 1; n >= 0; --n) to[db] = mfma16<IDT>(va, part[n], to[db]);
             }
+          }
+          if constexpr (IDT == PFA_I8) {
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) acc[db] += ta[db];
           }
         }
       }
@@ -536,8 +605,8 @@ tile_attn_kernel(AttnArgs a, int odt) {
         for (int k = 1; k < KS; ++k) {
           const float* o = (const float*)ring + (int64_t)(rg + RG * k) * W * 64 + lane;
           const float mo = o[0], mn = fmaxf(m, mo);
-          const float fa = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
-          const float fb = mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - mn);
+          const float fa = m == -INFINITY ? 0.f : exp2_p<IDT>(m - mn);
+          const float fb = mo == -INFINITY ? 0.f : exp2_p<IDT>(mo - mn);
           l = l * fa + o[64] * fb;
 #pragma unroll
           for (int db = 0; db < NDB; ++db)
@@ -549,14 +618,14 @@ tile_attn_kernel(AttnArgs a, int odt) {
     }
 
     if (ks == 0 && wmax >= 0) {
-      float inv = 1.f / l;
-      if constexpr (IDT == PFA_I8) inv *= a.v_scale[bh];
       bool bad = false;
+      const float inv = 1.f / l;
+      const float vs = IDT == PFA_I8 ? a.v_scale[bh] : 1.f;
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          acc[db][i] *= inv;
+          acc[db][i] = normalise<IDT>(acc[db][i], l, inv, vs);
           bad |= !(fabsf(acc[db][i]) <= 3.402823466e38f);
           if (l == 0.f) acc[db][i] = __builtin_nanf("");  // every score -inf
         }
@@ -621,12 +690,13 @@ static int launch_ks(const AttnArgs& a, int odt, hipStream_t s) {
 
 // Key splits by the number of 64-row blocks, against the chip's 256 CUs.
 // Measured on one box (us; key splits 1 / 2 / 4, D = 64 unless named):
-//   125 blocks, int8 causal, D = 32, T 1,000:   28.4 /  22.7 /  20.2
-//   188 blocks, f32 masked, T 1,500:           161.3 / 116.8 /  91.5
-//   188 blocks, bf16 masked, T 1,500:           72.0 /  52.7 /  45.8
-//   512 blocks, f16 causal, T 4,096:            86.4 /  75.7 /  88.3
-//   512 blocks, f32 causal, T 4,096:           201.9 / 212.6 / 228.7
-//   2,048 blocks, f16 causal, T 8,192:         365   / 408   / 532
+//   125 blocks, int8 causal, D = 32, T 1,000:   21.8 /  17.1 /  14.6
+//   188 blocks, f32 masked, T 1,500:           187.3 / 123.2 /  93.5
+//   188 blocks, bf16 masked, T 1,500:           68.0 /  47.4 /  41.1
+//   512 blocks, f16 causal, T 4,096:            82.2 /  73.5 /  85.1
+//   512 blocks, f32 causal, T 4,096:           230.6 / 239.3 / 248.7
+//   768 blocks, f16 causal, T 4,096:            99.2 /  98.4 / 122.6
+//   2,048 blocks, f16 causal, T 8,192:         368   / 428   / 553
 // Below one block per CU the splits fill the chip; up to three, two splits
 // even out the causal lengths of 16-bit rows (f32 rows are bound by the
 // matrix unit already); above, the whole blocks read each tile least often.

@@ -509,15 +509,20 @@ def _mfma_causal_ok(dtype: torch.dtype, D: int, *t4s: "_hip.Tensor4") -> bool:
 # Implicit causal bf16 rows on the tile kernel (pfa_sparse_attn_fwd) rather
 # than the structured kernel (pfa_shortlist_attn_fwd with a full window), by
 # the number of 64-row blocks.  The tile kernel splits keys over its waves when
-# the blocks do not fill the chip and keeps P at 16 more bits; the structured
-# kernel's larger blocks win once they do.  Measured on one box (us, structured
-# / tile):
-#   D = 64:  129 blocks, T 8,192: 160 / 68; 512, T 4,096: 76 / 63; 1,024, T 8,192:
-#            172 / 155; 2,048, T 2,048: 96 / 109; 4,096, T 32,768: 1,985 / 2,108
-#   D = 32:  129 blocks, T 8,192: 159 / 63; 2,048, T 4,096: 158 / 136; 4,096,
-#            T 32,768: 1,811 / 1,563
-#   D = 128: 129 blocks, T 8,192: 195 / 153; 254, T 4,096: 99 / 77; 511, T 4,096:
-#            118 / 132
+# the blocks do not fill the chip and keeps P at 24 bits, the structured kernel
+# at 8 (results of 1,500 tokens 1.56e-3 and 1.96e-3 from the 64-bit ones, of
+# which one rounding to bf16 is 1.55e-3).  The structured kernel's larger
+# blocks win once they fill the chip; up to the lines below, and for narrow
+# heads at any size, the tiles' bits come before that.  Measured on one box
+# (us, structured / tile):
+#   D = 64:  129 blocks, T 8,192: 151 / 64; 512, T 4,096: 81 / 70; 768, T 8,192:
+#            157 / 165; 1,024, T 8,192: 174 / 175; 2,048, T 2,048: 96 / 119;
+#            4,096, T 32,768: 1,855 / 2,287
+#   D = 32:  129 blocks, T 8,192: 141 / 54; 2,048, T 4,096: 141 / 175; 4,096,
+#            T 32,768: 1,424 / 1,666
+#   D = 16:  2,048 blocks, T 4,096: 135 / 159; 4,096, T 32,768: 1,369 / 1,471
+#   D = 128: 129 blocks, T 8,192: 185 / 144; 254, T 4,096: 93 / 79; 511, T 4,096:
+#            109 / 122
 _CAUSAL_TILE_BLOCKS = {16: None, 32: None, 64: 1024, 128: 256}
 
 
