@@ -365,7 +365,9 @@ int pfa_sparse_attn_fwd(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v,
                         const float* v_scale, void* stream);
 
 /* pfa_sparse_attn_fwd with a workspace of (N + 15) / 16 bytes (NULL for none),
- * which lets candidate rows share the keys of sixteen neighbours' lists. */
+ * which lets candidate rows share the keys of sixteen neighbours' lists.  Worth
+ * giving where the rows of one head of one batch row lie close: on average
+ * 16 tokens apart (f32) or 32 (other types), or less. */
 int pfa_sparse_attn_fwd_ws(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v,
                         int in_dtype, pfa_tensor4 out, int out_dtype, int H,
                         int64_t T, int D, const int32_t* token_idx,

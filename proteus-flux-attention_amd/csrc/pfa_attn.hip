@@ -125,21 +125,19 @@ sparse_attn_generic_kernel(AttnArgs a, int D) {
   for (int dd = lane; dd < D; dd += 64) store_f<ODT>(op + dd, (l == 0.f) ? __builtin_nanf("") : accs[dd] / l);
 }
 
-// Candidate rows on the union kernel: where its fixed cost (about 20 us: marking
-// and listing a workgroup's keys) is covered by the candidates (at most N * L),
-// the table's ranges are few and the rows of a head lie close (on average, of
-// one batch row): lists of distant rows share little.  Measured (us, rows /
-// union):
-//   T = 8,192, spacing 4, 16,400 rows: bf16 134 / 55, f32 143 / 86; spacing 1,
-//     65,500 rows: 449 / 162, 514 / 267
-//   T = 4,096, spacing 4, 8,200 rows: bf16 55 / 36, f32 66 / 42
-//   T = 32,768, spacing 4, 65,700 rows: bf16 515 / 298, f32 723 / 581
-//   T = 65,536, spacing 80, 6,600 rows: bf16 49 / 54, f32 73 / 99
-//   T = 20,000, spacing 33, 4,800 rows: bf16 50 / 83, f32 82 / 131
-//   T = 1,024, 2,100 rows: bf16 12 / 21, f32 11 / 22
+// Candidate rows on the union kernel, where the caller gave a workspace (rows of
+// a head that lie close enough to share their lists): where its fixed cost
+// (about 20 us: marking and listing a workgroup's keys) is covered by the
+// candidates (at most N * L) and the table's ranges are few.  Measured (us,
+// rows / union):
+//   T = 8,192, 16,384 rows x 512: bf16 132 / 49, f32 139 / 88; 65,536 rows:
+//     425 / 157, 514 / 290
+//   T = 4,096, 8,192 rows x 512: bf16 56 / 24, f32 67 / 40
+//   T = 32,768, 65,536 rows x 512: bf16 510 / 295, f32 732 / 592
+//   T = 1,024, 2,048 rows x 512: bf16 26 / 17, f32 26 / 23; of 256 entries: 12 / 21,
+//     11 / 22
 constexpr int64_t kUnionEntries = 3 << 20;
 constexpr int64_t kUnionKeys = 32768;
-constexpr int64_t kUnionSpacing = 16;
 
 template <int IDT, int ODT>
 static int launch_attn(AttnArgs a, int D, hipStream_t s) {
@@ -221,8 +219,7 @@ static int sparse_attn_run(pfa_tensor4 q, pfa_tensor4 k, pfa_tensor4 v, int in_d
   a.cand = cand; a.cand_stride = cand_stride; a.cand_len = cand_len; a.mask = mask; a.mask_dtype = mask_dtype;
   a.head_max = head_max_token; a.scale = scale; a.q_scale = q_scale; a.k_scale = k_scale; a.v_scale = v_scale;
   a.mode = cand ? kModeCand : (mask ? kModeMasked : kModeCausal);
-  a.flags = cand && !mask && N * cand_stride >= kUnionEntries && T <= kUnionKeys && T * H <= kUnionSpacing * N ? flags
-                                                                                                             : nullptr;
+  a.flags = cand && !mask && N * cand_stride >= kUnionEntries && T <= kUnionKeys ? flags : nullptr;
   hipStream_t s = as_stream(stream);
   if (in_dtype == PFA_F32 && out_dtype == PFA_F32) return launch_attn<PFA_F32, PFA_F32>(a, D, s);
   if (in_dtype == PFA_BF16 && out_dtype == PFA_BF16) return launch_attn<PFA_BF16, PFA_BF16>(a, D, s);

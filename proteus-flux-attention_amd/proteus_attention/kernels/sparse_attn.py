@@ -348,6 +348,29 @@ def build_packed_shortlist_candidates(
 # attention
 # ---------------------------------------------------------------------------
 
+# Candidate rows share their neighbours' lists (the union kernel) where the
+# rows of a head of one batch row lie, on average, at most this many tokens
+# apart: lists of distant rows share little, and f32 pays more for an unshared
+# key.  Measured on lists of 512 over windows of 256, anchors and prototypes (us,
+# rows / union):
+#   T = 8,192, spacing 16: bf16 129 / 58, f32 150 / 109; 32: 75 / 35, 95 / 71; 48:
+#     69 / 41, 92 / 109
+#   T = 16,384, spacing 16: bf16 79 / 44, f32 87 / 83; 24: 103 / 68, 121 / 168; 32:
+#     84 / 48, 100 / 138
+#   T = 32,768, spacing 8: bf16 266 / 157, f32 332 / 314; 16: 147 / 93, 172 / 182; 24:
+#     109 / 82, 130 / 184; 32: 153 / 105, 236 / 258
+#   T = 20,000, lists of 1,024, spacing 16: bf16 284 / 203, f32 350 / 334; 33:
+#     157 / 160, 229 / 247
+# (f16 and int8 as bf16)
+_UNION_SPACING = {torch.float32: 16}
+_UNION_SPACING_16 = 32
+
+
+def _union_rows(dtype: torch.dtype, T: int, heads: int, rows: int) -> bool:
+    """heads: the heads of every batch row together."""
+    return int(T) * int(heads) <= _UNION_SPACING.get(dtype, _UNION_SPACING_16) * int(rows)
+
+
 def _attn_launch(
     q4: "_hip.Tensor4",
     k4: "_hip.Tensor4",
@@ -369,15 +392,18 @@ def _attn_launch(
     scales: Tuple[Optional[torch.Tensor], Optional[torch.Tensor], Optional[torch.Tensor]],
     device: torch.device,
     n_rows_dev: Optional[torch.Tensor] = None,
+    batch: int = 1,
 ) -> None:
+    """batch: the batch rows, of H heads each, that the rows come from."""
     lib = _hip.lib()
     mask_tag = _hip.dtype_tag(mask.dtype) if mask is not None else 0
-    ws = _workspace((int(token_idx.numel()) + 15) // 16, device) if cand is not None and mask is None else None
+    N = int(token_idx.numel())
+    share = cand is not None and mask is None and _union_rows(in_dtype, T, int(batch) * int(H), N)
+    ws = _workspace((N + 15) // 16, device) if share else None
     with _hip.TIMER.timed("sparse_attn_fwd"):
         rc = lib.pfa_sparse_attn_fwd_ws(
         q4, k4, v4, _hip.dtype_tag(in_dtype), out4, _hip.dtype_tag(out_dtype), int(H), int(T), int(D),
-        _hip.ptr(token_idx), _hip.ptr(row_head), _hip.ptr(head_map), int(token_idx.numel()), _hip.ptr(n_rows_dev),
-        _hip.ptr(cand),
+        _hip.ptr(token_idx), _hip.ptr(row_head), _hip.ptr(head_map), N, _hip.ptr(n_rows_dev), _hip.ptr(cand),
         int(cand.stride(0)) if cand is not None else 0, _hip.ptr(cand_len), _hip.ptr(mask), mask_tag,
         _hip.ptr(head_max), float(scale), _hip.ptr(scales[0]), _hip.ptr(scales[1]), _hip.ptr(scales[2]),
         _hip.ptr(ws), ws.numel() if ws is not None else 0, _hip.stream_ptr(device))

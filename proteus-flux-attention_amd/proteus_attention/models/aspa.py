@@ -1849,12 +1849,12 @@ class AdaptiveSparseAttention(nn.Module):
             _sa._attn_launch(_hip.tensor4(q8[:, :, 0], H, "bthd"), _hip.tensor4(q8[:, :, 1], H, "bthd"),
                              _hip.tensor4(q8[:, :, 2], H, "bthd"), torch.int8, out4, qkv.dtype, H, T, D, token_idx,
                              row_head, heads, cand, None if causal else lens, None, None, 1.0 / math.sqrt(D),
-                             (scales[0], scales[1], scales[2]), device, n_rows_dev=rows_dev)
+                             (scales[0], scales[1], scales[2]), device, n_rows_dev=rows_dev, batch=B)
         else:
             _sa._attn_launch(_hip.tensor4(q5[:, :, 0], H, "bthd"), _hip.tensor4(q5[:, :, 1], H, "bthd"),
                              _hip.tensor4(q5[:, :, 2], H, "bthd"), qkv.dtype, out4, qkv.dtype, H, T, D, token_idx,
-                             row_head, heads, cand, None if causal else lens, None, None, 1.0 / math.sqrt(D), (None, None, None), device,
-                             n_rows_dev=rows_dev)
+                             row_head, heads, cand, None if causal else lens, None, None, 1.0 / math.sqrt(D),
+                             (None, None, None), device, n_rows_dev=rows_dev, batch=B)
         _record_backend("hip", device=str(device), tokens=T, rows=int(token_idx.numel()), L=L,
                         quantized=use_quant, candidates=True, structured=False)
         self._last_shortlist_backend_info = get_last_backend_info()
