@@ -241,6 +241,19 @@ class AdaptiveSparseAttention(nn.Module):
     _last_density = _lazy_stat("_last_density")
     _latency_ema = _lazy_stat("_latency_ema")
 
+    @property
+    def _last_shortlist_lengths(self) -> Optional[torch.Tensor]:
+        """Candidate counts of the last forward's rows.  Rows that take every
+        key 0..t have them in their tokens: counted when they are read."""
+        lens = self.__dict__.get("_shortlist_lengths")
+        if isinstance(lens, tuple):
+            lens = self.__dict__["_shortlist_lengths"] = lens[0] + 1
+        return lens
+
+    @_last_shortlist_lengths.setter
+    def _last_shortlist_lengths(self, lens) -> None:
+        self.__dict__["_shortlist_lengths"] = lens
+
     def __init__(self, config: ModelConfig):
         super().__init__()
         g = lambda name, default=None: getattr(config, name, default)  # noqa: E731
@@ -1238,7 +1251,7 @@ class AdaptiveSparseAttention(nn.Module):
 
     _GRAPH_STATE = ("_last_batch_size", "_current_alpha", "_token_keep_ratio_runtime", "_last_target_k",
                     "_last_gate_probs", "_last_token_similarity", "_last_token_blend", "_last_token_importance",
-                    "_last_token_mask", "_router_stats", "_proto_sums", "_last_shortlist_lengths",
+                    "_last_token_mask", "_router_stats", "_proto_sums", "_shortlist_lengths",
                     "_last_shortlist_backend_info", "_cached_active_mask", "_cached_packing", "_pending_summary",
                     "last_head_consensus", "last_router_reg", "last_aux_loss")
 
@@ -1834,11 +1847,12 @@ class AdaptiveSparseAttention(nn.Module):
                 rh = row_head.clamp(0, heads.numel() - 1) if rows_dev is not None else row_head
                 row_batch = (heads.index_select(0, rh) // H).to(torch.int32)
         if causal:
-            cand, lens = None, (token_idx + 1 if self.record_shortlist_lengths else None)
+            cand = lens = None
+            self._last_shortlist_lengths = (token_idx,)
         else:
             cand, lens = _sa._shortlist_build_device(token_idx, row_batch, T, L, local_w, stride, slots, sets,
                                                      n_rows_dev=rows_dev)
-        self._last_shortlist_lengths = lens
+            self._last_shortlist_lengths = lens
         out4 = _hip.tensor4(attn.view(B, T, H, D), H, "bthd")
         if use_quant:
             # Per-head int8 of the active heads (aspa.py:1258-1267) into an
@@ -1848,15 +1862,15 @@ class AdaptiveSparseAttention(nn.Module):
             scales = self._quantize_qkv(q5, B, T, heads, q8)
             _sa._attn_launch(_hip.tensor4(q8[:, :, 0], H, "bthd"), _hip.tensor4(q8[:, :, 1], H, "bthd"),
                              _hip.tensor4(q8[:, :, 2], H, "bthd"), torch.int8, out4, qkv.dtype, H, T, D, token_idx,
-                             row_head, heads, cand, None if causal else lens, None, None, 1.0 / math.sqrt(D),
+                             row_head, heads, cand, lens, None, None, 1.0 / math.sqrt(D),
                              (scales[0], scales[1], scales[2]), device, n_rows_dev=rows_dev, batch=B)
         else:
             _sa._attn_launch(_hip.tensor4(q5[:, :, 0], H, "bthd"), _hip.tensor4(q5[:, :, 1], H, "bthd"),
                              _hip.tensor4(q5[:, :, 2], H, "bthd"), qkv.dtype, out4, qkv.dtype, H, T, D, token_idx,
-                             row_head, heads, cand, None if causal else lens, None, None, 1.0 / math.sqrt(D),
+                             row_head, heads, cand, lens, None, None, 1.0 / math.sqrt(D),
                              (None, None, None), device, n_rows_dev=rows_dev, batch=B)
         _record_backend("hip", device=str(device), tokens=T, rows=int(token_idx.numel()), L=L,
-                        quantized=use_quant, candidates=True, structured=False)
+                        quantized=use_quant, candidates=cand is not None, structured=False)
         self._last_shortlist_backend_info = get_last_backend_info()
 
     def _quantize_qkv(self, q5: torch.Tensor, B: int, T: int, heads: torch.Tensor, dst5: torch.Tensor) -> torch.Tensor:
