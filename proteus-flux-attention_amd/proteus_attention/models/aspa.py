@@ -80,6 +80,19 @@ _SIDE_STREAMS: Dict[Tuple[int, str], torch.cuda.Stream] = {}
 _ONE_STREAM_ELEMS = {torch.bfloat16: 21 << 20, torch.float16: 6 << 20, torch.float32: 5 << 19}
 
 
+def _bytes_ever_allocated(device: torch.device) -> int:
+    return int(torch.cuda.memory_stats_as_nested_dict(device)["allocated_bytes"]["all"]["allocated"])
+
+
+def _capture_fits(allocated: int, device: torch.device) -> bool:
+    """Whether a capture whose forward makes `allocated` bytes of allocations
+    in all can take them from the driver, none returned to it.  Blocks come
+    from segments that may be half filled; a few small ones are open at a time."""
+    free, total = torch.cuda.mem_get_info(device)
+    share = int(torch.cuda.get_per_process_memory_fraction(device) * total)
+    return 2 * allocated + (64 << 20) <= min(free, share - torch.cuda.memory_reserved(device))
+
+
 def _side_stream(device: torch.device, role: str) -> torch.cuda.Stream:
     index = device.index if device.index is not None else torch.cuda.current_device()
     st = _SIDE_STREAMS.get((index, role))
@@ -1277,6 +1290,7 @@ class AdaptiveSparseAttention(nn.Module):
         try:
             side = _side_stream(device, "capture")
             side.wait_stream(torch.cuda.current_stream(device))
+            need = _bytes_ever_allocated(device)
             with torch.cuda.stream(side):
                 # warm-up: library handles, lazy allocations; with the output
                 # projection captured it runs here too, so that its GEMM sets
@@ -1285,6 +1299,7 @@ class AdaptiveSparseAttention(nn.Module):
                 if self._hip_graph_static_output:
                     self.dropout(self.proj(attn_w))
                 del attn_w
+            need = _bytes_ever_allocated(device) - need
             torch.cuda.current_stream(device).wait_stream(side)
             with torch.no_grad():
                 for n, b in self.named_buffers():
@@ -1301,20 +1316,19 @@ class AdaptiveSparseAttention(nn.Module):
             self._capture_keep = []
             # no garbage collection inside the capture: a dead object that
             # owns device resources (pinned host memory, events) would be
-            # freed while the stream captures, which is not allowed.  With the
-            # collector off none starts, so dead cycles need no collection
-            # first (24 ms in a process with a torch heap).  The allocator's
-            # cache is kept where the card has as much free memory besides
-            # (torch.cuda.graph always empties it: 4 ms, and the buffers around
-            # the capture are then allocated from the driver again); a capture
-            # cannot release cached blocks itself.
+            # freed while the stream captures, which is not allowed.  A capture
+            # cannot release cached blocks either: where the memory that the
+            # warm-up forward took is not free besides, dead cycles are
+            # collected (24 ms in a process with a torch heap) and the
+            # allocator's cache is emptied first (4 ms, and the buffers around
+            # the capture are then allocated from the driver again).
+            torch.cuda.synchronize(device)
+            if not _capture_fits(need, device):
+                gc.collect()
+                torch.cuda.empty_cache()
             gc_was_on = gc.isenabled()
             gc.disable()
             try:
-                torch.cuda.synchronize(device)
-                cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
-                if torch.cuda.mem_get_info(device)[0] < cached:
-                    torch.cuda.empty_cache()
                 side = _side_stream(device, "capture")
                 with torch.cuda.stream(side):
                     graph.capture_begin(pool=self._hip_graph_pool)
