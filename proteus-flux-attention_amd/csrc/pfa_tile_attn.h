@@ -288,7 +288,10 @@ tile_attn_kernel(AttnArgs a, int odt) {
       wmax = max(wmax, __shfl_xor(wmax, o, 64));
       wmin = min(wmin, __shfl_xor(wmin, o, 64));
     }
-    const int kmax = __builtin_amdgcn_readfirstlane(MASKED ? a.head_max[hp] : smax);  // last key
+    // the last key, of those there are: below 0 no key at all (no score, NaN
+    // rows, as in the row kernel), and the loads stay at key 0
+    const int kmax = min(__builtin_amdgcn_readfirstlane(MASKED ? a.head_max[hp] : smax), (int)a.T - 1);
+    const int kload = max(kmax, 0);
     wmax = __builtin_amdgcn_readfirstlane(wmax);
     wmin = __builtin_amdgcn_readfirstlane(wmin);
     const int nstep = kmax / (TK * KS) + 1;
@@ -320,7 +323,7 @@ tile_attn_kernel(AttnArgs a, int odt) {
         for (int j = 0; j < kJ; ++j) {
           // 16-bit tiles of D = 128: the second 64-dim half after the first
           const int row = row0 + kRowStep * j % TK, elem = (elem0 ^ (kFlip * (j & 1))) + 64 * (kRowStep * j / TK);
-          const int key = min((st * KS + sub) * TK + row, kmax);
+          const int key = min((st * KS + sub) * TK + row, kload);
           const uint32_t dst = stage + sub * C::kTileBytes + 4096 * j;
           if (off32) {
             lds_dma16_s(kb, ((uint32_t)key * (uint32_t)a.k.s_t + elem) * (uint32_t)sizeof(IT), dst);
@@ -339,7 +342,7 @@ tile_attn_kernel(AttnArgs a, int odt) {
       for (int j = 0; j < kReg; ++j) {
         const int n = tid + 256 * j;
         const int c = n % CW, row = (n / CW) % TK, sub = (n / (CW * TK)) % KS;
-        const int key = min((st * KS + sub) * TK + row, kmax);
+        const int key = min((st * KS + sub) * TK + row, kload);
         const int e = 8 * (c & (D / 8 - 1));
         const IT* src = n / (CW * TK * KS) ? vb + (int64_t)key * a.v.s_t + e : kb + (int64_t)key * a.k.s_t + e;
         regs[j] = *reinterpret_cast<const uint2*>(src);
