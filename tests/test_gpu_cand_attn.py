@@ -1,6 +1,8 @@
 """Candidate attention over the union of sixteen lists (pfa_cand_attn.h): lists
-of several ranges and flushes, shared and unshared, unsorted, repeated or out
-of range, against the row kernel and the oracle in 64 bits."""
+of several ranges, shared and unshared, unsorted, repeated or out of range, some
+attended by the union kernel and some left by it to the row kernel, against the
+oracle in 64 bits.  (More keys than the kernel lists at a time:
+test_gpu_union_lists.py.)"""
 from __future__ import annotations
 
 import pytest

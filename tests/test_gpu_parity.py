@@ -1524,8 +1524,9 @@ def test_dropin_mha_fallbacks_match_torch(dev):
 def test_operator_causal_branch_mfma_vs_oracle(dev, BH, T, p, D):
     """aspa_sparse_attention without candidates or mask (each active row
     attends to keys 0..t, sparse_attn.py:1016-1043) in bf16, D = 16, 32, 64
-    or 128, runs the MFMA causal tiles; every active row against f32 causal
-    attention, inactive rows zero."""
+    or 128, runs on matrix-core tiles (these sizes the tile kernel; larger ones
+    the structured kernel, test_gpu_tile_paths.py); every active row against f32
+    causal attention, inactive rows zero."""
     from proteus_attention.kernels.sparse_attn import aspa_sparse_attention, get_last_backend_info
 
     _say(f"operator causal mfma BH={BH} T={T} p={p} D={D}")
@@ -1548,7 +1549,7 @@ def test_operator_causal_branch_mfma_vs_oracle(dev, BH, T, p, D):
 def test_module_force_dense_mfma_vs_oracle(dev, B, T, dt, keep):
     """subquad mode (force-dense, aspa.py:1624-1677): the attention output
     equals causal attention of the module's own projected and rotated
-    q/k/v (bf16 on the MFMA causal tiles, f32 on the row kernel).  With
+    q/k/v (both on the tile kernel).  With
     token sparsity (keep) only the kept tokens' rows are attended and the
     others are exactly zero: the reference's dense output times the token
     mask (aspa.py:1841-1842)."""

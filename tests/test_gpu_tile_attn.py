@@ -35,8 +35,9 @@ def _mask(T, dt, g):
 @pytest.mark.parametrize("D", [16, 32, 64, 128])
 @pytest.mark.parametrize("masked", [False, True])
 def test_tile_attention_edges(dt, D, masked):
-    """Lengths around a tile, heads that share a row block, one row, and
-    enough rows for each key split (blocks of 64 rows <= 256, <= 768, above)."""
+    """Lengths around a tile, heads that share a row block, one row, and at 32
+    and 64 dims enough rows for each key split (blocks of 64 rows <= 256, <= 768,
+    above; every width, over many tiles: test_gpu_attn_precision.py)."""
     from proteus_attention.kernels.sparse_attn import aspa_sparse_attention
 
     dev = torch.device("cuda:0")
