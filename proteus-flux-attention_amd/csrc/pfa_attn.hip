@@ -150,9 +150,10 @@ static int launch_attn(AttnArgs a, int D, hipStream_t s) {
   vec = vec && al(a.q, ies) && al(a.k, ies) && al(a.v, ies) && al(a.out, oes);
   // Rows of one head share keys: causal and masked rows on tiles of them,
   // candidate rows on the union of sixteen lists, both on the matrix cores.
-  // bf16 inputs with f32 results would need P at more than the 16 bits those
-  // keep: rows, as for a mask beside candidates.  The row kernel behind the
-  // union kernel takes the rows it leaves.
+  // bf16 inputs with f32 results go by rows (the tiles add bf16 products to the
+  // running sum one by one, for results of 16 bits), as does a mask beside
+  // candidates.  The row kernel behind the union kernel takes the rows it
+  // leaves.
   if (vec && a.T < INT32_MAX / 2 && !(IDT == PFA_BF16 && ODT == PFA_F32)) {
     if (a.mode != kModeCand && (a.mode != kModeMasked || a.T >= 4)) {
       if constexpr (IDT == PFA_F32) return tile_attn_launch_f32(a, ODT, D, s);

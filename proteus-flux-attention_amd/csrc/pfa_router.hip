@@ -1263,12 +1263,10 @@ static void launch_accum(const void* x, int64_t n_tok, int C, int G, const float
   else proto_accum_kernel<DT, 64><<<n_parts, kEmaThreads, 0, s>>>((const ET*)x, n_tok, C, G, gp, per, partial);
 }
 
-// Telemetry partials (n_blocks, 8) summed column-wise in f64 into out[8]:
-// thread t owns column t % 8 and the blocks t/8 + 128k; each pass issues
-// eight independent loads before adding them, and the 128 per-column
-// partials are then added in a fixed tree order (deterministic).
-// The statistics' sums in a fixed order, whatever the block size: 1024
-// virtual threads, each a column (of 8) of every 128th row, then a tree.
+// Telemetry partials (n_blocks, 8) summed column-wise in f64 into out[8], in
+// an order that does not depend on the block size: virtual thread t of 1024
+// owns column t % 8 and the rows t/8 + 128k, eight independent loads before
+// their sums; the 128 sums of a column are then added as a tree.
 __device__ __forceinline__ void stats_reduce_block(const float* __restrict__ stats, int n_blocks,
                                                    double* __restrict__ out, double* part) {
   for (int t = threadIdx.x; t < 1024; t += blockDim.x) {

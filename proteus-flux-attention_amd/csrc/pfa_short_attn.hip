@@ -88,9 +88,9 @@ struct ShortArgs {
   const float* vsc;
   // work the anchor pass takes over from separate passes (kFuse* bits)
   int fuse;
-  // head dim D (16, 32 or 64) and cmask = D/8 - 1: rows narrower than 64
-  // are attended as 64-wide rows whose q dims past D are zero (their K/V
-  // tile chunks hold copies of the row's own chunks, see dma_tile)
+  // head dim D and cmask = D/8 - 1 (D <= 64).  Of rows of 16 dims the score
+  // product's 32 are read: q is zero past D, and those K chunks hold copies of
+  // the row's own (see dma_tile32).
   int dh;
   uint32_t cmask;
   __device__ __forceinline__ float head_scale_log2(int bh) const {

@@ -401,8 +401,8 @@ prefix_sb_prefix(int nsb, int64_t SB, int K, const uint64_t* __restrict__ skey,
 // S(64j - 1) = top-K(R[s] U Q) best first, Q = the tokens of superblock s
 // before the block, best first (the superblock's sorted list with its later
 // positions dropped, an ordered compaction), by a merge-path co-rank.
-// LDS: R[s], Q and P (cap keys each), P's positions, index-sorted copy and
-// ranks (cap each).
+// LDS: R[s], Q and P (cap keys each), P's positions and ranks (cap each); P
+// sorted by index takes the place of R[s].
 template <bool SORT>
 __global__ void __launch_bounds__(256)
 prefix_block_walk(const float* __restrict__ scores, int64_t T, int64_t stride, int nb, int64_t SB, int nsb, int K,

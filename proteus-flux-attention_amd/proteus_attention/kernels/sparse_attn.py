@@ -515,9 +515,9 @@ def _shortlist_attn_structured(
     return lengths
 
 
-# Head dims of the structured MFMA kernel: rows of 16 or 32 elements are
-# attended as 64-wide rows whose q dims past D are zero, rows of 128 as two
-# 64-dim halves of each tile.
+# Head dims of the structured MFMA kernel.  Its tile rows hold 64 dims: of rows
+# of 16 or 32 only the chunks that a product reads are filled, rows of 128 take
+# two halves.
 STRUCTURED_HEAD_DIMS = (16, 32, 64, 128)
 
 

@@ -1713,9 +1713,10 @@ class AdaptiveSparseAttention(nn.Module):
 
     def _shortlist_plan(self, B: int, T: int, alpha: float, dtype: torch.dtype,
                         sims: Optional[bool] = None) -> Dict[str, Any]:
-        """Shortlist sizes of this forward (aspa.py:1175-1210) and whether the
-        structured kernel serves it (bf16, D=64, no row truncated).  `sims`:
-        whether the router gives prototype similarities (default: whether
+        """Shortlist sizes of this forward (aspa.py:1175-1210), whether the
+        structured kernel can serve it ("fits": bf16, D in
+        STRUCTURED_HEAD_DIMS, no row truncated) and whether it does
+        ("structured").  `sims`: whether the router gives prototype similarities (default: whether
         this forward's router gave them)."""
         D = self.d_head
         if sims is None:
