@@ -1716,8 +1716,8 @@ class AdaptiveSparseAttention(nn.Module):
         """Shortlist sizes of this forward (aspa.py:1175-1210), whether the
         structured kernel can serve it ("fits": bf16, D in
         STRUCTURED_HEAD_DIMS, no row truncated) and whether it does
-        ("structured").  `sims`: whether the router gives prototype similarities (default: whether
-        this forward's router gave them)."""
+        ("structured").  `sims`: whether the router gives prototype
+        similarities (default: whether this forward's router gave them)."""
         D = self.d_head
         if sims is None:
             sims = self._last_token_similarity is not None
